@@ -64,6 +64,10 @@ struct kate_batch {
     int64_t* d_zoff = nullptr;
     double* d_z = nullptr;
     double* d_norms = nullptr;
+    kate::ZItem* d_zitems = nullptr;
+    uint32_t* d_zfirst = nullptr;
+    double* d_zpart = nullptr;
+    uint32_t nzitems = 0;
     kate::BatchTask* d_tasks = nullptr;
     uint32_t* d_counters = nullptr;  // done[npasses], next, err
     kate::PassArgs* d_passes = nullptr;
@@ -87,7 +91,8 @@ void release(kate_batch* b)
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
     if (b->graph) (void)hipGraphDestroy(b->graph);
     void* ptrs[] = {b->d_states, b->d_circ_off, b->d_nq, b->d_nq_int, b->d_zoff, b->d_z, b->d_norms, b->d_tasks,
-                    b->d_counters, b->d_passes, b->d_micro, b->d_ops, b->d_coef, b->d_raw};
+                    b->d_counters, b->d_passes, b->d_micro, b->d_ops, b->d_coef, b->d_raw,
+                    b->d_zitems, b->d_zfirst, b->d_zpart};
     for (void* p : ptrs) (void)hipFree(p);
     for (auto& e : b->ev)
         if (e) (void)hipEventDestroy(e);
@@ -106,6 +111,10 @@ kate::BatchArgs args(kate_batch* b)
     a.zoff = b->d_zoff;
     a.z = b->d_z;
     a.norms = b->d_norms;
+    a.zitems = b->d_zitems;
+    a.nzitems = b->nzitems;
+    a.zfirst = b->d_zfirst;
+    a.zpart = b->d_zpart;
     a.count = b->count;
     a.tasks = b->d_tasks;
     a.ntasks = b->ntasks;
@@ -234,6 +243,15 @@ int kate_batch_create(const kate_program* programs, int32_t count, const kate_op
             }
         }
     b->ntasks = (uint32_t)tasks.size();
+    std::vector<kate::ZItem> zitems;
+    std::vector<uint32_t> zfirst;
+    for (uint32_t c = 0; c < (uint32_t)count; c++) {
+        zfirst.push_back((uint32_t)zitems.size());
+        const uint32_t blocks = b->nq_int[c] > kate::kZBlockBits ? 1u << (b->nq_int[c] - kate::kZBlockBits) : 1u;
+        for (uint32_t t = 0; t < blocks; t++) zitems.push_back(kate::ZItem{c, t});
+    }
+    zfirst.push_back((uint32_t)zitems.size());
+    b->nzitems = (uint32_t)zitems.size();
 
     int rc = KATE_OK;
     auto step = [&](hipError_t e, const char* what) {
@@ -247,6 +265,9 @@ int kate_batch_create(const kate_program* programs, int32_t count, const kate_op
     step(hipMalloc((void**)&b->d_z, std::max<int64_t>(1, b->zlen) * sizeof(double)), "hipMalloc(z)");
     step(hipMalloc((void**)&b->d_norms, b->count * sizeof(double)), "hipMalloc(norms)");
     step(hipMalloc((void**)&b->d_counters, (b->npasses + 2) * sizeof(uint32_t)), "hipMalloc(counters)");
+    step(hipMalloc((void**)&b->d_zpart, (size_t)b->nzitems * kate::kZRow * sizeof(double)), "hipMalloc(z sums)");
+    if (rc == KATE_OK) rc = put(&b->d_zitems, zitems);
+    if (rc == KATE_OK) rc = put(&b->d_zfirst, zfirst);
     if (rc == KATE_OK) rc = put(&b->d_circ_off, circ_off);
     if (rc == KATE_OK) rc = put(&b->d_nq, b->nq);
     if (rc == KATE_OK) rc = put(&b->d_nq_int, b->nq_int);

@@ -33,46 +33,77 @@ __global__ __launch_bounds__(256) void k_batch_ones(Cx<R>* __restrict__ states, 
     if (c < count) states[circ_off[c]] = Cx<R>{(R)1, (R)0};
 }
 
-// Per circuit (one workgroup each): norm and <Z_q> for every qubit, FP64,
-// fixed summation order.  Amplitude i = it*256 + tid.
+// <Z_q> and norms of a batch, level 1: workgroup w reduces the amplitudes
+// [tile << kZBlockBits, ...) of circuit item.circuit to {sum |a|^2, and for
+// each of the low kZBlockBits index bits the sum over the amplitudes with
+// that bit set} (FP64, fixed order).  Bound by the read of the states: one
+// workgroup per circuit, as this was first split, left a 20-qubit circuit to
+// one CU (256 complex64 circuits of 10-20 qubits: 2.82 ms, 240 MB; blocks of
+// 2^14 amplitudes and a sum over blocks: 0.09 ms).
 template <typename R>
 __global__ __launch_bounds__(256) void k_batch_z(const Cx<R>* __restrict__ states, const uint64_t* __restrict__ circ_off,
-                                                 const int32_t* __restrict__ nq, const int32_t* __restrict__ nq_int,
-                                                 const int64_t* __restrict__ zoff, double* __restrict__ z,
-                                                 double* __restrict__ norms)
+                                                 const int32_t* __restrict__ nq_int, const ZItem* __restrict__ items,
+                                                 double* __restrict__ part)
 {
-    __shared__ double lds[4];
-    const uint32_t c = blockIdx.x, tid = threadIdx.x;
-    const Cx<R>* st = states + circ_off[c];
-    const int n = nq[c];
-    const uint64_t iters = 1ull << (nq_int[c] - 8);
-    double tot = 0.0, hi[24];
+    constexpr int H = kZBlockBits - 8;  // index bits of the loops
+    const uint32_t tid = threadIdx.x;
+    const ZItem item = items[blockIdx.x];
+    const Cx<R>* __restrict__ st = states + circ_off[item.circuit] + ((uint64_t)item.tile << kZBlockBits);
+    const int bits = nq_int[item.circuit];
+    const uint32_t iters = 1u << ((bits < kZBlockBits ? bits : kZBlockBits) - 8);
+    double val[1 + H + 8];
 #pragma unroll
-    for (int q = 0; q < 24; q++) hi[q] = 0.0;
-    for (uint64_t it = 0; it < iters; it++) {
+    for (int q = 0; q < 1 + H; q++) val[q] = 0.0;
+#pragma unroll 4
+    for (uint32_t it = 0; it < iters; it++) {
         const Cx<R> a = st[(it << 8) | tid];
         const double p = (double)a.re * (double)a.re + (double)a.im * (double)a.im;
-        tot += p;
+        val[0] += p;
 #pragma unroll
-        for (int q = 0; q < 24; q++)
-            if (q + 8 < n && ((it >> q) & 1ull)) hi[q] += p;
+        for (int q = 0; q < H; q++)
+            if ((it >> q) & 1u) val[1 + q] += p;
     }
-    const double total = block_sum(tot, lds);
-    double* out = z + zoff[c];
-    for (int q = 0; q < n; q++) {
-        double s1;
-        if (q < 8) {
-            s1 = block_sum(((tid >> q) & 1u) ? tot : 0.0, lds);
-        } else {
-            double h = 0.0;
 #pragma unroll
-            for (int j = 0; j < 24; j++)
-                if (j == q - 8) h = hi[j];
-            s1 = block_sum(h, lds);
+    for (int q = 0; q < 8; q++) val[1 + H + q] = ((tid >> q) & 1u) ? val[0] : 0.0;
+    __shared__ double wpart[4][1 + H + 8];
+#pragma unroll
+    for (int j = 0; j < 1 + H + 8; j++) {
+        const double s = wave_sum(val[j]);
+        if ((tid & 63u) == 0) wpart[tid >> 6][j] = s;
+    }
+    __syncthreads();
+    if (tid < 1 + H + 8) {
+        // row: total, bits 0..7 (threads), bits 8.. (loop)
+        const int at = tid == 0 ? 0 : (tid <= (uint32_t)H ? (int)tid + 8 : (int)tid - H);
+        part[(uint64_t)blockIdx.x * kZRow + at] =
+            (wpart[0][tid] + wpart[1][tid]) + (wpart[2][tid] + wpart[3][tid]);
+    }
+}
+
+// Level 2, one workgroup per circuit: wave w takes the sums of qubits w, w+4,
+// ... over the circuit's blocks (an index bit above the block's is a bit of
+// the block number), lanes over the blocks.
+__global__ __launch_bounds__(256) void k_batch_zfin(const double* __restrict__ part, const uint32_t* __restrict__ first,
+                                                    const int32_t* __restrict__ nq, const int64_t* __restrict__ zoff,
+                                                    double* __restrict__ z, double* __restrict__ norms)
+{
+    const uint32_t c = blockIdx.x, lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    const uint32_t r0 = first[c], rows = first[c + 1] - r0;
+    const int n = nq[c];
+    double total = 0.0;
+    for (uint32_t r = lane; r < rows; r += 64) total += part[(uint64_t)(r0 + r) * kZRow];
+    total = wave_sum(total);
+    for (int q = (int)w; q < n; q += 4) {
+        double s1 = 0.0;
+        for (uint32_t r = lane; r < rows; r += 64) {
+            const double* row = part + (uint64_t)(r0 + r) * kZRow;
+            if (q < kZBlockBits) s1 += row[1 + q];
+            else if ((r >> (q - kZBlockBits)) & 1u) s1 += row[0];
         }
-        if (tid == 0) out[q] = (total - 2.0 * s1) / total;
+        s1 = wave_sum(s1);
+        if (lane == 0) z[zoff[c] + q] = (total - 2.0 * s1) / total;
     }
-    if (tid == 0) norms[c] = total;
+    if (threadIdx.x == 0) norms[c] = total;
 }
 
 // ---- initialisation --------------------------------------------------------
@@ -116,161 +147,227 @@ __global__ __launch_bounds__(256) void k_scale(Cx<R>* __restrict__ st, uint64_t 
 
 // ---- deterministic reductions ------------------------------------------------
 
-// Level 0 of the amplitude sums: a block reduces 4096 amplitudes (tile index
-// it*256 + tid) to one record {total, S1[bit 0..11]}.
-// With GATHER the amplitude of index i is read at offset M(i), M linear over
-// GF(2) with columns gm.col[] (a state whose last permutation passes have
-// not run yet: M maps each final index to where its amplitude still is).
+// State offsets of index bits for a read through a GF(2)-linear map: the
+// amplitude of index i is at the XOR of col[] over the set bits of i (a state
+// whose last permutation passes have not run yet).
 struct GatherMap {
     uint64_t col[kMaxQubits];
 };
 
+// Kate's amplitude sums: sum_x a_x and, for every index bit q, the sum over
+// the x with bit q set, in two launches whatever the size.  Level 1: block b
+// of G = gridDim.x (a power of two) reads the 4096-amplitude chunks b + i*G,
+// 16 loads in flight per thread.  Index bits: 0-7 thread, 8-11 load, then
+// log2(G) bits of b, then the bits of i.  Per chunk each thread adds its 16
+// amplitudes to the total, the four load-bit sums and, uniformly over the
+// block, the sums of the set bits of i; the thread bits and the waves are
+// reduced once per block.  Column c of the sums is part[c * G + b]: 0 the
+// total, 1-8 the thread bits, 9-12 the load bits, 13.. the bits of i.
+// Bound by the read (proba_state call, 30 qubits complex128: 17.2 GB in 3.29
+// -> 2.86 ms, 6.0 TB/s; 28 qubits complex64 0.86 -> 0.39 ms) or, up to about
+// 22 qubits, by its two launches (20 qubits 48 -> 24 us): a workgroup per
+// chunk that reduced 26 values for 4096 amplitudes, and levels of 256 rows
+// reduced value by value in one workgroup, cost more than the loads.
+constexpr int kSumCols = 13 + kSumIterBits;
+
 template <typename R, bool GATHER>
-__global__ __launch_bounds__(256) void k_sums0(const Cx<R>* __restrict__ st, double* __restrict__ rec, GatherMap gm)
+__global__ __launch_bounds__(256) void k_ampsums(const Cx<R>* __restrict__ st, uint64_t chunks, GatherMap gm,
+                                                 double* __restrict__ part)
 {
-    const uint32_t tid = threadIdx.x;
-    const uint64_t base = (uint64_t)blockIdx.x << 12;
-    uint64_t gbase = 0;
-    if constexpr (GATHER) {
-        const uint32_t blk = blockIdx.x;
+    const uint32_t tid = threadIdx.x, G = gridDim.x;
+    constexpr int V = 5 + kSumIterBits;
+    double vr[V], vi[V];  // total, 4 load bits, bits of i
 #pragma unroll
-        for (int j = 0; j < kMaxQubits - 12; j++)
-            if ((blk >> j) & 1u) gbase ^= gm.col[12 + j];
+    for (int j = 0; j < V; j++) vr[j] = vi[j] = 0.0;
+    uint64_t tbase = 0;
+    if constexpr (GATHER) {
 #pragma unroll
         for (int j = 0; j < 8; j++)
-            if ((tid >> j) & 1u) gbase ^= gm.col[j];
+            if ((tid >> j) & 1u) tbase ^= gm.col[j];
     }
-    double tr = 0, ti = 0, hr[4] = {0, 0, 0, 0}, hi[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int it = 0; it < 16; it++) {
-        uint64_t off = base + ((uint64_t)it << 8) + tid;
+    uint32_t i = 0;
+    for (uint64_t c = blockIdx.x; c < chunks; c += G, i++) {
+        Cx<R> a[16];
+        uint64_t gbase = tbase;
         if constexpr (GATHER) {
-            off = gbase;
+            for (int j = 0; (c >> j) != 0; j++)
+                if ((c >> j) & 1ull) gbase ^= gm.col[12 + j];
+        }
+#pragma unroll
+        for (int it = 0; it < 16; it++) {
+            uint64_t off = (c << 12) + ((uint64_t)it << 8) + tid;
+            if constexpr (GATHER) {
+                off = gbase;
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if ((it >> j) & 1) off ^= gm.col[8 + j];
+            }
+            a[it] = st[off];
+        }
+        double cr = 0, ci = 0;
+#pragma unroll
+        for (int it = 0; it < 16; it++) {
+            const double re = (double)a[it].re, im = (double)a[it].im;
+            cr += re;
+            ci += im;
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                if ((it >> j) & 1) off ^= gm.col[8 + j];
+                if ((it >> j) & 1) {
+                    vr[1 + j] += re;
+                    vi[1 + j] += im;
+                }
         }
-        const Cx<R> a = st[off];
-        tr += (double)a.re;
-        ti += (double)a.im;
+        vr[0] += cr;
+        vi[0] += ci;
 #pragma unroll
-        for (int b = 0; b < 4; b++)
-            if ((it >> b) & 1) {
-                hr[b] += (double)a.re;
-                hi[b] += (double)a.im;
+        for (int j = 0; j < kSumIterBits; j++)
+            if ((i >> j) & 1u) {
+                vr[5 + j] += cr;
+                vi[5 + j] += ci;
             }
     }
-    // Per wave (butterflies, no barrier): the totals, the sums over lanes
-    // with lane bit q set (q < 6) and the loop-bit sums; one barrier, then
-    // thread 0 adds the four waves in a fixed order.  Bits 6 and 7 of the
-    // amplitude index are the wave index, so their sums are the totals of
-    // waves 1, 3 and of waves 2, 3.
-    constexpr int V = 2 + 12 + 8;
-    double val[V];
-    val[0] = wave_sum(tr);
-    val[1] = wave_sum(ti);
-#pragma unroll
-    for (int q = 0; q < 6; q++) {
-        const bool on = (tid >> q) & 1u;
-        val[2 + 2 * q] = wave_sum(on ? tr : 0.0);
-        val[3 + 2 * q] = wave_sum(on ? ti : 0.0);
-    }
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-        val[14 + 2 * b] = wave_sum(hr[b]);
-        val[15 + 2 * b] = wave_sum(hi[b]);
-    }
-    __shared__ double part[4][V];
+    __shared__ double wpart[4][2 * (V + 8)];
     const uint32_t w = tid >> 6;
-    if ((tid & 63u) == 0) {
 #pragma unroll
-        for (int j = 0; j < V; j++) part[w][j] = val[j];
+    for (int j = 0; j < V + 6; j++) {
+        double re, im;
+        if (j < V) {
+            re = vr[j];
+            im = vi[j];
+        } else {  // thread bit j - V
+            const bool on = (tid >> (j - V)) & 1u;
+            re = on ? vr[0] : 0.0;
+            im = on ? vi[0] : 0.0;
+        }
+        re = wave_sum(re);
+        im = wave_sum(im);
+        if ((tid & 63u) == 0) {
+            wpart[w][2 * j] = re;
+            wpart[w][2 * j + 1] = im;
+            if (j == 0) {  // thread bits 6 and 7 are the wave number
+                wpart[w][2 * (V + 6)] = (w & 1u) ? re : 0.0;
+                wpart[w][2 * (V + 6) + 1] = (w & 1u) ? im : 0.0;
+                wpart[w][2 * (V + 7)] = (w & 2u) ? re : 0.0;
+                wpart[w][2 * (V + 7) + 1] = (w & 2u) ? im : 0.0;
+            }
+        }
     }
     __syncthreads();
-    if (tid == 0) {
-        double* out = rec + (uint64_t)blockIdx.x * 26;
-        auto all = [&](int j) { return (part[0][j] + part[1][j]) + (part[2][j] + part[3][j]); };
-        out[0] = all(0);
-        out[1] = all(1);
-        for (int q = 0; q < 6; q++) {
-            out[2 + 2 * q] = all(2 + 2 * q);
-            out[3 + 2 * q] = all(3 + 2 * q);
-        }
-        out[14] = part[1][0] + part[3][0];  // index bit 6
-        out[15] = part[1][1] + part[3][1];
-        out[16] = part[2][0] + part[3][0];  // index bit 7
-        out[17] = part[2][1] + part[3][1];
-        for (int b = 0; b < 4; b++) {
-            out[18 + 2 * b] = all(14 + 2 * b);
-            out[19 + 2 * b] = all(15 + 2 * b);
-        }
+    if (tid < 2 * (V + 8)) {
+        const double s = (wpart[0][tid] + wpart[1][tid]) + (wpart[2][tid] + wpart[3][tid]);
+        const int j = (int)tid >> 1;
+        const int col = j == 0 ? 0 : (j < V ? j + 8 : j - V + 1);
+        if (G > 1 || col <= 12) part[2 * ((uint64_t)col * G + blockIdx.x) + (tid & 1u)] = s;
     }
 }
 
-// Level >= 1: a block reduces 2^C records {total, S1[0..K)} (one per thread)
-// into {total, S1[0..K), S1[K..K+C)}.
-__global__ __launch_bounds__(256) void k_sums_rec(const double* __restrict__ in, int K, int C, double* __restrict__ out)
+// Level 2: workgroup 0 adds the total's column, workgroup 1 + q the column of
+// index bit q (or, for a bit of the block number, the totals of the blocks
+// with it set).
+__global__ __launch_bounds__(256) void k_ampsums_fin(const double* __restrict__ part, uint32_t G, int gbits,
+                                                     double* __restrict__ out)
 {
     __shared__ double lds[4];
-    const uint32_t tid = threadIdx.x;
-    const bool valid = tid < (1u << C);
-    const uint64_t r = ((uint64_t)blockIdx.x << C) + tid;
-    const int win = 2 * (1 + K), wout = 2 * (1 + K + C);
-    const double* src = in + r * (uint64_t)win;
-    double* dst = out + (uint64_t)blockIdx.x * (uint64_t)wout;
-    const double tr = valid ? src[0] : 0.0, ti = valid ? src[1] : 0.0;
-    for (int f = 0; f < win; f++) {
-        const double s = block_sum(valid ? src[f] : 0.0, lds);
-        if (tid == 0) dst[f] = s;
+    const int q = (int)blockIdx.x - 1;
+    const int bbit = (q >= 12 && q < 12 + gbits) ? q - 12 : -1;
+    const int col = q < 0 || bbit >= 0 ? 0 : (q < 12 ? q + 1 : q - 12 - gbits + 13);
+    const double* __restrict__ p = part + 2 * (uint64_t)col * G;
+    double re = 0, im = 0;
+#pragma unroll 4
+    for (uint32_t r = threadIdx.x; r < G; r += 256) {
+        const bool on = bbit < 0 || ((r >> bbit) & 1u);
+        re += on ? p[2 * (uint64_t)r] : 0.0;
+        im += on ? p[2 * (uint64_t)r + 1] : 0.0;
     }
-    for (int c = 0; c < C; c++) {
-        const bool on = valid && ((tid >> c) & 1u);
-        double s = block_sum(on ? tr : 0.0, lds);
-        if (tid == 0) dst[win + 2 * c] = s;
-        s = block_sum(on ? ti : 0.0, lds);
-        if (tid == 0) dst[win + 2 * c + 1] = s;
+    re = block_sum(re, lds);
+    im = block_sum(im, lds);
+    if (threadIdx.x == 0) {
+        out[2 * blockIdx.x] = re;
+        out[2 * blockIdx.x + 1] = im;
     }
 }
 
-// Level 0 of the Z sums: a block reduces 4096 amplitudes to MB signed sums.
-template <typename R, int MB>
-__global__ __launch_bounds__(256) void k_z0(const Cx<R>* __restrict__ st, const uint64_t* __restrict__ masks, int m,
-                                            double* __restrict__ part)
+// Walsh-Hadamard transform of 16 values over their 4 index bits.
+__device__ __forceinline__ void wht16(double (&v)[16])
 {
-    const uint32_t tid = threadIdx.x;
-    const uint64_t base = (uint64_t)blockIdx.x << 12;
-    double acc[MB];
-    uint32_t sgn[MB];
-    uint64_t mk[MB];
 #pragma unroll
-    for (int j = 0; j < MB; j++) {
-        acc[j] = 0.0;
-        mk[j] = j < m ? masks[j] : 0ull;
-        sgn[j] = (uint32_t)(__popcll((base | tid) & mk[j]) & 1);
-    }
+    for (int b = 0; b < 4; b++)
 #pragma unroll
-    for (int it = 0; it < 16; it++) {
-        const Cx<R> a = st[base + ((uint64_t)it << 8) + tid];
-        const double p = (double)a.re * (double)a.re + (double)a.im * (double)a.im;
-#pragma unroll
-        for (int j = 0; j < MB; j++) {
-            const uint32_t f = sgn[j] ^ (uint32_t)(__popcll(((uint64_t)it << 8) & mk[j]) & 1);
-            acc[j] += f ? -p : p;
+        for (int s = 0; s < 16; s++) {
+            if ((s >> b) & 1) continue;
+            const double x = v[s], y = v[s | (1 << b)];
+            v[s] = x + y;
+            v[s | (1 << b)] = x - y;
         }
-    }
-    // wave butterflies, then one barrier and a fixed-order sum of the waves
-    __shared__ double wpart[4][MB];
+}
+
+struct ZMaskArg {
+    uint64_t m[kZMasks];
+};
+
+// Z strings: sum_x |a_x|^2 (-1)^popcount(x & mask) for up to kZMasks masks in
+// one read of the state.  Each 4096-amplitude chunk is transformed by a
+// Walsh-Hadamard transform of |a|^2 (three 16-point steps in registers with
+// two exchanges through LDS: 12 additions per amplitude), after which the sum
+// of a mask over the chunk is one entry, mask & 4095, with the sign of the
+// mask on the chunk's number; thread j keeps mask j's sum.  The cost no
+// longer depends on the number of masks, and the kernel is bound by the read
+// (41 masks, 28 qubits complex64: three reads of 16 signed sums each 2.09 ms,
+// this 0.40 ms, 5.4 TB/s; 20 qubits 137 -> 21 us a call).  LDS: 32 KiB, XOR swizzle of the low 4 index bits with
+// the next 4, so each exchange's 16 lanes hit 16 distinct 8-byte slots.
+template <typename R>
+__global__ __launch_bounds__(256) void k_zwht(const Cx<R>* __restrict__ st, uint64_t chunks, ZMaskArg mk, int m,
+                                              double* __restrict__ part)
+{
+    __shared__ double w[4096];
+    const uint32_t tid = threadIdx.x, lo = tid & 15u, hi = tid >> 4;
+    const uint64_t mask = tid < (uint32_t)m ? mk.m[tid & (kZMasks - 1)] : 0ull;
+    const uint32_t mlow = (uint32_t)mask & 4095u;
+    double acc = 0.0;
+    for (uint64_t c = blockIdx.x; c < chunks; c += gridDim.x) {
+        double v[16];
 #pragma unroll
-    for (int j = 0; j < MB; j++) acc[j] = wave_sum(acc[j]);
-    if ((tid & 63u) == 0) {
+        for (int it = 0; it < 16; it++) {
+            const Cx<R> a = st[(c << 12) + ((uint64_t)it << 8) + tid];
+            v[it] = (double)a.re * (double)a.re + (double)a.im * (double)a.im;
+        }
+        wht16(v);  // index bits 8..11
 #pragma unroll
-        for (int j = 0; j < MB; j++) wpart[tid >> 6][j] = acc[j];
+        for (int r = 0; r < 16; r++) w[((uint32_t)r << 8) | (hi << 4) | (lo ^ hi)] = v[r];
+        __syncthreads();
+        // index bits 0..3: this thread holds indices (hi, lo, r)
+#pragma unroll
+        for (int r = 0; r < 16; r++) v[r] = w[(hi << 8) | (lo << 4) | ((uint32_t)r ^ lo)];
+        wht16(v);
+#pragma unroll
+        for (int r = 0; r < 16; r++) w[(hi << 8) | (lo << 4) | ((uint32_t)r ^ lo)] = v[r];
+        __syncthreads();
+        // index bits 4..7: indices (hi, r, lo)
+#pragma unroll
+        for (int r = 0; r < 16; r++) v[r] = w[(hi << 8) | ((uint32_t)r << 4) | (lo ^ (uint32_t)r)];
+        wht16(v);
+#pragma unroll
+        for (int r = 0; r < 16; r++) w[(hi << 8) | ((uint32_t)r << 4) | (lo ^ (uint32_t)r)] = v[r];
+        __syncthreads();
+        if (tid < (uint32_t)m) {
+            const double x = w[(mlow & ~15u) | ((mlow ^ (mlow >> 4)) & 15u)];
+            acc += (__popcll((c << 12) & mask) & 1) ? -x : x;
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    if (tid < (uint32_t)MB) {
-        double* out = part + (uint64_t)blockIdx.x * MB;
-        out[tid] = (wpart[0][tid] + wpart[1][tid]) + (wpart[2][tid] + wpart[3][tid]);
-    }
+    if (tid < (uint32_t)m) part[(uint64_t)tid * gridDim.x + blockIdx.x] = acc;
+}
+
+// Level 2: workgroup j adds the G partial sums of mask j.
+__global__ __launch_bounds__(256) void k_rows_fin(const double* __restrict__ part, uint32_t G, double* __restrict__ out)
+{
+    __shared__ double lds[4];
+    const double* __restrict__ p = part + (uint64_t)blockIdx.x * G;
+    double a = 0.0;
+#pragma unroll 4
+    for (uint32_t r = threadIdx.x; r < G; r += 256) a += p[r];
+    a = block_sum(a, lds);
+    if (threadIdx.x == 0) out[blockIdx.x] = a;
 }
 
 // Level 0 of <a|b> = sum conj(a_i) b_i (FP64): a block reduces 4096
@@ -438,8 +535,8 @@ int launch_batch(int dtype, const BatchArgs& a, void* stream)
                            a.circ_off, a.count);
         int e = launch_batch_kernel_f64(a, s);
         if (e) return e;
-        hipLaunchKernelGGL(k_batch_z<double>, dim3(a.count), dim3(256), 0, s, (const Cx<double>*)a.states, a.circ_off,
-                           a.nq, a.nq_int, a.zoff, a.z, a.norms);
+        hipLaunchKernelGGL(k_batch_z<double>, dim3(a.nzitems), dim3(256), 0, s, (const Cx<double>*)a.states, a.circ_off,
+                           a.nq_int, a.zitems, a.zpart);
     } else {
         hipLaunchKernelGGL(k_batch_init<float>, dim3(grid_for(a.total_amps)), dim3(256), 0, s, (Cx<float>*)a.states,
                            a.total_amps, a.circ_off, a.count);
@@ -447,9 +544,10 @@ int launch_batch(int dtype, const BatchArgs& a, void* stream)
                            a.circ_off, a.count);
         int e = launch_batch_kernel_f32(a, s);
         if (e) return e;
-        hipLaunchKernelGGL(k_batch_z<float>, dim3(a.count), dim3(256), 0, s, (const Cx<float>*)a.states, a.circ_off,
-                           a.nq, a.nq_int, a.zoff, a.z, a.norms);
+        hipLaunchKernelGGL(k_batch_z<float>, dim3(a.nzitems), dim3(256), 0, s, (const Cx<float>*)a.states, a.circ_off,
+                           a.nq_int, a.zitems, a.zpart);
     }
+    hipLaunchKernelGGL(k_batch_zfin, dim3(a.count), dim3(256), 0, s, a.zpart, a.zfirst, a.nq, a.zoff, a.z, a.norms);
     return (int)hipGetLastError();
 }
 
@@ -543,12 +641,28 @@ int launch_scale(int dtype, void* state, int nq_int, double factor, void* stream
     return (int)hipGetLastError();
 }
 
+namespace {
+
+// log2 of the level-1 workgroups of the amplitude and Z sums: a chunk each up
+// to 2^11 workgroups (eight per CU), then up to 16 chunks each, then more
+// workgroups (30 qubits complex128: a fixed grid of 2^11 left the last of its
+// three rounds over the chip two thirds full).
+int sum_grid_bits(int nq_int)
+{
+    const int cbits = nq_int - 12;
+    if (cbits <= 11) return cbits;
+    return std::max(11, cbits - kSumIterBits);
+}
+
+}  // namespace
+
 uint64_t reduce_scratch_doubles(int nq_int)
 {
-    // level-0 records (26 doubles per 4096 amplitudes) twice over, plus the
-    // Z partials (16 per 4096), with slack for the small levels.
+    // the level-1 sums, and the rows of the overlap (4 per 4096 amplitudes
+    // and 4 per 4096 rows)
     const uint64_t chunks = 1ull << (nq_int > 12 ? nq_int - 12 : 0);
-    return chunks * 26 * 2 + chunks * 16 * 2 + 4096;
+    const uint64_t g = 1ull << sum_grid_bits(std::max(nq_int, 12));
+    return std::max<uint64_t>(g * std::max(2 * kSumCols, kZMasks), chunks * 5) + 4096;
 }
 
 int launch_amp_sums(int dtype, const void* state, int nq_int, double* d_scratch, double* d_out, void* stream,
@@ -556,70 +670,46 @@ int launch_amp_sums(int dtype, const void* state, int nq_int, double* d_scratch,
 {
     hipStream_t s = (hipStream_t)stream;
     if (nq_int < 12 || nq_int > kMaxQubits) return (int)hipErrorInvalidValue;
-    uint64_t count = 1ull << (nq_int - 12);
-    double* a = count == 1 ? d_out : d_scratch;
-    double* b = d_scratch + count * 26 + 64;
+    const uint64_t chunks = 1ull << (nq_int - 12);
+    const int gbits = sum_grid_bits(nq_int);
+    const dim3 g(1u << gbits), t(256);
+    double* part = gbits ? d_scratch : d_out;  // one workgroup's columns are the result
     GatherMap gm{};
     if (gather_cols) {
-        const uint64_t lim = nq_int >= 64 ? ~0ull : ((1ull << nq_int) - 1ull);
+        const uint64_t lim = (1ull << nq_int) - 1ull;
         for (int q = 0; q < nq_int; q++) {
             if (gather_cols[q] & ~lim) return (int)hipErrorInvalidValue;  // offsets stay inside the state
             gm.col[q] = gather_cols[q];
         }
     }
+#define AS(R, GA) hipLaunchKernelGGL((k_ampsums<R, GA>), g, t, 0, s, (const Cx<R>*)state, chunks, gm, part)
     if (dtype == 0) {
-        if (gather_cols)
-            hipLaunchKernelGGL((k_sums0<double, true>), dim3((unsigned)count), dim3(256), 0, s,
-                               (const Cx<double>*)state, a, gm);
-        else
-            hipLaunchKernelGGL((k_sums0<double, false>), dim3((unsigned)count), dim3(256), 0, s,
-                               (const Cx<double>*)state, a, gm);
+        if (gather_cols) AS(double, true);
+        else AS(double, false);
     } else {
-        if (gather_cols)
-            hipLaunchKernelGGL((k_sums0<float, true>), dim3((unsigned)count), dim3(256), 0, s,
-                               (const Cx<float>*)state, a, gm);
-        else
-            hipLaunchKernelGGL((k_sums0<float, false>), dim3((unsigned)count), dim3(256), 0, s,
-                               (const Cx<float>*)state, a, gm);
+        if (gather_cols) AS(float, true);
+        else AS(float, false);
     }
-    int K = 12;
-    while (count > 1) {
-        int C = 0;
-        while (C < 8 && (1ull << (C + 1)) <= count) C++;
-        const uint64_t blocks = count >> C;
-        double* dst = (blocks == 1) ? d_out : b;
-        hipLaunchKernelGGL(k_sums_rec, dim3((unsigned)blocks), dim3(256), 0, s, a, K, C, dst);
-        K += C;
-        count = blocks;
-        std::swap(a, b);
-        if (blocks == 1) break;
-    }
+#undef AS
+    if (gbits) hipLaunchKernelGGL(k_ampsums_fin, dim3((unsigned)nq_int + 1), t, 0, s, d_scratch, 1u << gbits, gbits, d_out);
     return (int)hipGetLastError();
 }
 
-int launch_zsums(int dtype, const void* state, int nq_int, const uint64_t* d_masks, int count, double* d_scratch,
+int launch_zsums(int dtype, const void* state, int nq_int, const uint64_t* masks, int count, double* d_scratch,
                  double* d_out, void* stream)
 {
     hipStream_t s = (hipStream_t)stream;
-    if (nq_int < 12 || count < 1 || count > 16) return (int)hipErrorInvalidValue;
+    if (nq_int < 12 || nq_int > kMaxQubits || count < 1 || count > kZMasks) return (int)hipErrorInvalidValue;
     const uint64_t chunks = 1ull << (nq_int - 12);
-    double* a = chunks == 1 ? d_out : d_scratch;
-    double* b = d_scratch + chunks * 16 + 64;
+    const uint32_t G = 1u << sum_grid_bits(nq_int);
+    ZMaskArg mk{};
+    std::copy(masks, masks + count, mk.m);
+    double* part = G == 1 ? d_out : d_scratch;
     if (dtype == 0)
-        hipLaunchKernelGGL((k_z0<double, 16>), dim3((unsigned)chunks), dim3(256), 0, s, (const Cx<double>*)state,
-                           d_masks, count, a);
+        hipLaunchKernelGGL(k_zwht<double>, dim3(G), dim3(256), 0, s, (const Cx<double>*)state, chunks, mk, count, part);
     else
-        hipLaunchKernelGGL((k_z0<float, 16>), dim3((unsigned)chunks), dim3(256), 0, s, (const Cx<float>*)state,
-                           d_masks, count, a);
-    uint64_t rows = chunks;
-    while (rows > 1) {
-        const uint64_t blocks = (rows + 4095) / 4096;
-        double* dst = blocks == 1 ? d_out : b;
-        hipLaunchKernelGGL(k_rowsum, dim3((unsigned)blocks), dim3(256), 0, s, a, rows, 16, dst);
-        rows = blocks;
-        std::swap(a, b);
-        if (blocks == 1) break;
-    }
+        hipLaunchKernelGGL(k_zwht<float>, dim3(G), dim3(256), 0, s, (const Cx<float>*)state, chunks, mk, count, part);
+    if (G > 1) hipLaunchKernelGGL(k_rows_fin, dim3((unsigned)count), dim3(256), 0, s, d_scratch, G, d_out);
     return (int)hipGetLastError();
 }
 

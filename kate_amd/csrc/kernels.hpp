@@ -28,6 +28,16 @@ struct BatchTask {
     uint32_t pad[2];
 };
 
+// <Z_q> of a batch: a block of 2^kZBlockBits amplitudes of one circuit per
+// workgroup, one row of kZRow sums each.
+constexpr int kZBlockBits = 14;
+constexpr int kZRow = 1 + kZBlockBits;
+
+struct ZItem {
+    uint32_t circuit;
+    uint32_t tile;
+};
+
 struct BatchArgs {
     void* states;
     uint64_t total_amps;
@@ -37,6 +47,10 @@ struct BatchArgs {
     const int64_t* zoff;
     double* z;
     double* norms;
+    const ZItem* zitems;     // every block of every circuit, in circuit order
+    uint32_t nzitems;
+    const uint32_t* zfirst;  // [count + 1]: first block of each circuit
+    double* zpart;           // [nzitems * kZRow]
     uint32_t count;
     const BatchTask* tasks;
     uint32_t ntasks;
@@ -75,6 +89,11 @@ int launch_init_product(int dtype, void* state, int nq_int, const double* d_fact
 // Multiplies every amplitude by `factor`.
 int launch_scale(int dtype, void* state, int nq_int, double factor, void* stream);
 
+// Z strings per launch_zsums call.
+constexpr int kZMasks = 64;
+// Chunk-number bits a level-1 workgroup of the amplitude sums loops over.
+constexpr int kSumIterBits = 4;
+
 // Sizes of the scratch buffer (in doubles) the reductions need.
 uint64_t reduce_scratch_doubles(int nq_int);
 // Amplitude sums: out[0..1] = sum of all amplitudes, out[2+2q..] = sum of the
@@ -85,8 +104,10 @@ uint64_t reduce_scratch_doubles(int nq_int);
 // passes have not run).
 int launch_amp_sums(int dtype, const void* state, int nq_int, double* d_scratch, double* d_out, void* stream,
                     const uint64_t* gather_cols = nullptr);
-// out[j] = sum_x |a_x|^2 (-1)^popcount(x & masks[j]) for j < count (FP64).
-int launch_zsums(int dtype, const void* state, int nq_int, const uint64_t* d_masks, int count, double* d_scratch,
+// out[j] = sum_x |a_x|^2 (-1)^popcount(x & masks[j]) for j < count <= kZMasks
+// (FP64; masks: host array).  d_out of both sums is device memory or
+// device-visible pinned host memory.
+int launch_zsums(int dtype, const void* state, int nq_int, const uint64_t* masks, int count, double* d_scratch,
                  double* d_out, void* stream);
 
 // d_out[0..3] = {Re, Im} of <a|b> = sum conj(a_i) b_i, sum |a_i|^2,

@@ -7,7 +7,7 @@
 //     input and queues the request (first come, first served);
 //   * the scheduler plans queued requests, admits the oldest ones whose
 //     footprint (state + plan + reduction scratch) fits the free arena,
-//     enqueues init, every pass, the Z reduction and the result copy on the
+//     enqueues init, every pass and the Z reduction on the
 //     next stream of the pool, and keeps going: requests that arrive while
 //     others run are admitted as soon as memory frees up, and their kernels
 //     overlap on the device through the different streams;
@@ -100,7 +100,7 @@ struct Request {
     bool planned = false;
     // arena ranges
     uint64_t off = 0, bytes = 0;
-    uint64_t o_state = 0, o_micro = 0, o_ops = 0, o_coef = 0, o_raw = 0, o_scratch = 0, o_out = 0, o_masks = 0,
+    uint64_t o_state = 0, o_micro = 0, o_ops = 0, o_coef = 0, o_raw = 0, o_scratch = 0,
              o_factors = 0, o_state2 = 0, o_scatter = 0;
     std::vector<float> coef32;
     int stream = -1;
@@ -180,8 +180,6 @@ uint64_t layout(kate_server* s, Request& r)
     r.o_coef = take(r.plan.coef.size() * (s->amp / 2));
     r.o_raw = take(r.plan.raw.size() * sizeof(uint32_t));
     r.o_scratch = take(kate::reduce_scratch_doubles(r.plan.nq_int) * sizeof(double));
-    r.o_out = take(64 * sizeof(double));
-    r.o_masks = take(16 * sizeof(uint64_t));
     r.o_factors = take(4 * (uint64_t)r.plan.nq_int * sizeof(double));
     if (!r.plan.scatter_args.empty()) {  // out-of-place passes: a second state buffer
         r.o_state2 = take((1ull << r.plan.nq_int) * s->amp);
@@ -214,7 +212,6 @@ int launch_request(kate_server* s, Request& r)
     if (!r.plan.raw.empty())
         SV(hipMemcpyAsync(base + r.o_raw, r.plan.raw.data(), r.plan.raw.size() * sizeof(uint32_t),
                           hipMemcpyHostToDevice, st));
-    SV(hipMemcpyAsync(base + r.o_masks, r.masks.data(), r.masks.size() * sizeof(uint64_t), hipMemcpyHostToDevice, st));
     if (!r.plan.scatter_args.empty())
         SV(hipMemcpyAsync(base + r.o_scatter, r.plan.scatter_args.data(),
                           r.plan.scatter_args.size() * sizeof(kate::ScatterArgs), hipMemcpyHostToDevice, st));
@@ -253,10 +250,10 @@ int launch_request(kate_server* s, Request& r)
         if (k) return k;
         if (pa.scatter) std::swap(state, other);
     }
-    k = kate::launch_zsums(s->opt.dtype, state, r.plan.nq_int, (const uint64_t*)(base + r.o_masks),
-                           (int)r.masks.size(), (double*)(base + r.o_scratch), (double*)(base + r.o_out), st);
+    // the sums go straight to the request's pinned slot
+    k = kate::launch_zsums(s->opt.dtype, state, r.plan.nq_int, r.masks.data(), (int)r.masks.size(),
+                           (double*)(base + r.o_scratch), r.host_out, st);
     if (k) return k;
-    SV(hipMemcpyAsync(r.host_out, base + r.o_out, 16 * sizeof(double), hipMemcpyDeviceToHost, st));
     SV(hipEventRecord(r.done_ev, st));
 #undef SV
     return 0;

@@ -166,7 +166,7 @@ struct kate_sim {
     uint32_t* d_raw = nullptr;
     double* d_scratch = nullptr;
     double* d_out = nullptr;
-    uint64_t* d_masks = nullptr;
+    double* h_out = nullptr;  // pinned: the reductions write their results here
     double* d_factors = nullptr;
     std::vector<double> h_factors;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -177,6 +177,10 @@ struct kate_sim {
 };
 
 namespace {
+
+// Doubles of kate_sim::h_out: the amplitude sums of kMaxQubits qubits, or
+// kZMasks Z sums.
+constexpr size_t kSlots = 2 + 2 * (size_t)kate::kMaxQubits + kate::kZMasks;
 
 template <typename T>
 int upload(T** dst, const std::vector<T>& src, hipStream_t s)
@@ -203,7 +207,7 @@ void release(kate_sim* s)
     (void)hipFree(s->d_raw);
     (void)hipFree(s->d_scratch);
     (void)hipFree(s->d_out);
-    (void)hipFree(s->d_masks);
+    (void)hipHostFree(s->h_out);
     (void)hipFree(s->d_factors);
     for (auto& e : s->ev)
         if (e) (void)hipEventDestroy(e);
@@ -289,21 +293,22 @@ int init_product(kate_sim* s, const double* tp)
 }
 
 // Kate's proba_state from the amplitude sums (HIPcode/simulator.hpp:519-536).
-int measure(kate_sim* s, double* out)
+// `done` (nullable) is recorded behind the sums.
+int measure(kate_sim* s, double* out, hipEvent_t done = nullptr)
 {
     // with the trailing passes pending, amplitude i is still at offset
     // trail_inv(i)
     const uint64_t* gather = s->pending ? s->plan.trail_inv.data() : nullptr;
-    int e = kate::launch_amp_sums(s->dtype, s->d_state, s->nq_int, s->d_scratch, s->d_out, s->stream, gather);
+    int e = kate::launch_amp_sums(s->dtype, s->d_state, s->nq_int, s->d_scratch, s->h_out, s->stream, gather);
     if (e) return fail(KATE_ERR_HIP, std::string("measure launch: ") + hipGetErrorString((hipError_t)e));
-    std::vector<double> sums(2 + 2 * (size_t)s->nq_int);
-    KATE_HIP(hipMemcpyAsync(sums.data(), s->d_out, sums.size() * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+    if (done) KATE_HIP(hipEventRecord(done, s->stream));
     KATE_HIP(hipStreamSynchronize(s->stream));
+    const double* sums = s->h_out;
     const int n = s->nq;
     const double den = std::pow(1.4142135623730951, (double)n);
     const double pi = 3.1415926535897932384626433;
     for (int q = 0; q < n; q++) {
-        const double s1r = sums[2 + 2 * (size_t)q], s1i = sums[3 + 2 * (size_t)q];
+        const double s1r = sums[2 + 2 * q], s1i = sums[3 + 2 * q];
         const double s0r = sums[0] - s1r, s0i = sums[1] - s1i;
         const double nn = den * den;
         const double a0 = (s0r * den) / nn, b0 = (den * s0i) / nn;
@@ -331,15 +336,13 @@ int measure(kate_sim* s, double* out)
 int zsums(kate_sim* s, const std::vector<uint64_t>& masks, std::vector<double>& out)
 {
     out.assign(masks.size(), 0.0);
-    for (size_t b = 0; b < masks.size(); b += 16) {
-        const int cnt = (int)std::min<size_t>(16, masks.size() - b);
-        KATE_HIP(hipMemcpyAsync(s->d_masks, masks.data() + b, cnt * sizeof(uint64_t), hipMemcpyHostToDevice, s->stream));
-        int e = kate::launch_zsums(s->dtype, s->d_state, s->nq_int, s->d_masks, cnt, s->d_scratch, s->d_out, s->stream);
+    for (size_t b = 0; b < masks.size(); b += kate::kZMasks) {
+        const int cnt = (int)std::min<size_t>(kate::kZMasks, masks.size() - b);
+        int e = kate::launch_zsums(s->dtype, s->d_state, s->nq_int, masks.data() + b, cnt, s->d_scratch, s->h_out,
+                                   s->stream);
         if (e) return fail(KATE_ERR_HIP, std::string("zsum launch: ") + hipGetErrorString((hipError_t)e));
-        double h[16];
-        KATE_HIP(hipMemcpyAsync(h, s->d_out, sizeof(h), hipMemcpyDeviceToHost, s->stream));
         KATE_HIP(hipStreamSynchronize(s->stream));
-        for (int j = 0; j < cnt; j++) out[b + (size_t)j] = h[j];
+        for (int j = 0; j < cnt; j++) out[b + (size_t)j] = s->h_out[j];
     }
     return KATE_OK;
 }
@@ -553,7 +556,7 @@ int kate_sim_create(const kate_program* program, const kate_options* options, ka
     }
     step(hipMalloc((void**)&s->d_scratch, kate::reduce_scratch_doubles(s->nq_int) * sizeof(double)), "hipMalloc(scratch)");
     step(hipMalloc((void**)&s->d_out, (2 + 2 * (size_t)s->nq_int + 64) * sizeof(double)), "hipMalloc(out)");
-    step(hipMalloc((void**)&s->d_masks, 16 * sizeof(uint64_t)), "hipMalloc(masks)");
+    step(hipHostMalloc((void**)&s->h_out, kSlots * sizeof(double), 0), "hipHostMalloc(out)");
     step(hipMalloc((void**)&s->d_factors, 4 * (size_t)s->nq_int * sizeof(double)), "hipMalloc(factors)");
     if (rc == KATE_OK) rc = upload(&s->d_micro, s->plan.micro, s->stream);
     if (rc == KATE_OK) rc = upload(&s->d_ops, s->plan.ops, s->stream);
@@ -700,11 +703,11 @@ size_t execute_pass_count(const kate_sim* s)
 
 int execute_impl(kate_sim* s, const double* tp_in, double* tp_out, hipEvent_t* pass_ev, uint64_t* pass_tiles)
 {
-    KATE_HIP(hipEventRecord(s->ev[0], s->stream));
     // |0...0> is made by the first pass itself (no init pass over HBM) unless
     // there is no pass to make it
     s->pending = false;  // the state is made afresh
     const bool fused_init = !tp_in && !s->plan.passes.empty();
+    if (!fused_init) KATE_HIP(hipEventRecord(s->ev[0], s->stream));
     int rc = KATE_OK;
     if (tp_in) rc = init_product(s, tp_in);
     else if (!fused_init) rc = kate::launch_init_basis(s->dtype, s->d_state, s->nq_int, 0, s->stream);
@@ -718,12 +721,10 @@ int execute_impl(kate_sim* s, const double* tp_in, double* tp_out, hipEvent_t* p
     s->pending = n_run < s->plan.passes.size();
     KATE_HIP(hipEventRecord(s->ev[2], s->stream));
     std::vector<double> tmp(2 * (size_t)s->nq);
-    rc = measure(s, tp_out ? tp_out : tmp.data());
+    rc = measure(s, tp_out ? tp_out : tmp.data(), s->ev[3]);
     if (rc) return rc;
-    KATE_HIP(hipEventRecord(s->ev[3], s->stream));
-    KATE_HIP(hipEventSynchronize(s->ev[3]));
     float a = 0, b = 0, c = 0;
-    KATE_HIP(hipEventElapsedTime(&a, s->ev[0], s->ev[1]));
+    if (!fused_init) KATE_HIP(hipEventElapsedTime(&a, s->ev[0], s->ev[1]));
     KATE_HIP(hipEventElapsedTime(&b, s->ev[1], s->ev[2]));
     KATE_HIP(hipEventElapsedTime(&c, s->ev[2], s->ev[3]));
     s->last.init_ms = a;
