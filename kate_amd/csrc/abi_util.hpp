@@ -10,4 +10,7 @@ namespace kate {
 int set_error(int code, const std::string& msg);
 std::string program_from_abi(const kate_program* in, Program& p);
 std::string plan_options(const kate_options& opt, PlanOptions& po);
+// Whether every shape and form is left to the planner, so that it may use
+// streamed passes (PlanOptions::stream).
+bool may_stream(const kate_options& opt, const PlanOptions& po);
 }  // namespace kate

@@ -585,6 +585,9 @@ int launch_pass(int dtype, int tile_bits, void* state, int nq_int, const PassArg
 {
     if (pa.tile_bits != tile_bits || nq_int < tile_bits || nq_int - tile_bits > 31 || pa.nrest > nq_int - tile_bits)
         return (int)hipErrorInvalidValue;
+    if (pa.stream)
+        return dtype == 0 ? launch_stream_f64(tile_bits, state, pa, dp, stream)
+                          : launch_stream_f32(tile_bits, state, pa, dp, stream);
     if (dtype == 0) return launch_pass_f64(tile_bits, state, nq_int, pa, dp, stream);
     return launch_pass_f32(tile_bits, state, nq_int, pa, dp, stream);
 }

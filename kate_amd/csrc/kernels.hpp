@@ -13,9 +13,10 @@ struct DevPlan {
     const MicroStep* micro;
     const MicroOp* ops;
     const void* coef;  // complex of the state's precision
-    const uint32_t* raw;  // matrix-core operands
+    const uint32_t* raw;  // matrix-core operands, streamed op codes
     void* dst = nullptr;                  // a gate pass with PassArgs::scatter writes this buffer
     const ScatterArgs* scatter = nullptr; // through these offsets (device memory)
+    const Phase* phases = nullptr;        // streamed passes
 };
 
 struct BatchTask {

@@ -639,7 +639,9 @@ __device__ __forceinline__ uint64_t rest_base(const PassArgs& pa, uint64_t blk)
 
 static_assert(offsetof(MicroStep, op0_code) == 2 && offsetof(MicroStep, coef) == 12 &&
                   offsetof(MicroStep, op_begin) == 4 && offsetof(MicroStep, op_count) == 8 &&
-                  offsetof(MicroStep, tbyte) == 112 && offsetof(MicroStep, pbyte) == 160,
+                  offsetof(MicroStep, pbyte) == 16 && offsetof(MicroStep, wbyte) == 32 &&
+                  offsetof(MicroStep, wflip) == 48 && offsetof(MicroStep, tbyte) == 52 &&
+                  offsetof(MicroStep, phase_coef) == 100,
               "step_addressing reads MicroStep as 32-bit words");
 
 // Addressing of an SK_REG micro-step for this thread: op range, the LDS
@@ -654,11 +656,11 @@ __device__ __forceinline__ void step_addressing(const MicroStep* __restrict__ ms
     op_begin = w[1];
     op_count = w[2];
 #pragma unroll
-    for (int k = 0; k < 4; k++) o[k] = w[40 + k];
+    for (int k = 0; k < 4; k++) o[k] = w[4 + k];
     b = 0;
 #pragma unroll
     for (int i = 0; i < TB - NB; i++)
-        if ((tid >> i) & 1u) b ^= w[28 + i];
+        if ((tid >> i) & 1u) b ^= w[13 + i];
 }
 
 template <typename R>
@@ -1037,6 +1039,313 @@ void k_pass(Cx<R>* __restrict__ state, PassArgs pa,
 {
     __shared__ Cx<R> tile[1 << TB];
     tile_pass<R, TB, WIDE, NB, LIGHT>(state, pa, blockIdx.x, tile, micro, ops, coef, raw, dst, sa);
+}
+
+// ---- streamed passes -----------------------------------------------------------
+//
+// k_stream runs the passes of 1-qubit, CNOT and CRk gates (PassArgs::stream).
+// Each register step is a stream of three ops -- a rotation along any register
+// direction, a 16-entry diagonal, a phase of the thread -- and writes its
+// registers back through a linear map, so CNOTs inside a step cost nothing
+// and diagonal gates collect into one product.  A CRk needs only one of its
+// qubits in registers: the other one's value is a bit of the thread index or of
+// the tile's offset, and the phases of all of them are one factor per
+// register bit, looked up in 16-entry tables.  The 300 CRk of a 25-qubit QFT
+// then fit the 3 passes its Hadamards need (14 with both qubits in registers:
+// 5.05 -> 1.33 ms complex128; a copy of the state is 0.2 ms a pass).  Bound by
+// the latency of the ops' operands with two workgroups of four waves per CU:
+// scalar loads of rotations and diagonals (their cache lines are fetched ahead
+// of the step: 45 % of a step waited on them), table lookups (read one op ahead).
+
+// [[1, -it], [-it, 1]] on every pair (s, s ^ D) in place; the member with the
+// lowest bit of D set comes out divided by 1 + t^2 (u = t / (1 + t^2)).
+template <int D, typename R>
+__device__ __forceinline__ void rotate(Cx<R> (&v)[16], R t, R u)
+{
+    constexpr int LOW = D & -D;
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+        if (s & LOW) continue;
+        v[s].re = fmar(t, v[s ^ D].im, v[s].re);
+        v[s].im = fmar(-t, v[s ^ D].re, v[s].im);
+        v[s ^ D].re = fmar(u, v[s].im, v[s ^ D].re);
+        v[s ^ D].im = fmar(-u, v[s].re, v[s ^ D].im);
+    }
+}
+
+// Registers with parity(s & M) ^ P times h.
+template <int M, int P, typename R>
+__device__ __forceinline__ void phase(Cx<R> (&v)[16], Cx<R> h)
+{
+#pragma unroll
+    for (int s = 0; s < 16; s++)
+        if ((popc4(s & M) & 1) ^ P) v[s] = cmul(h, v[s]);
+}
+
+// The ops of a streamed step, their codes four to a word.  `pt`: the thread
+// tables of its SC_PHASE ops (NT: bits of the thread index), read one op
+// ahead; `tile_phase`: the tile's factors of the same ops.
+template <typename R, int NT>
+__device__ __forceinline__ void stream_ops(Cx<R> (&v)[16], const uint32_t* __restrict__ codes,
+                                           const Cx<R>* __restrict__ cf, const Cx<R>* __restrict__ pt,
+                                           const Cx<R>* tile_phase, uint32_t phases)
+{
+    constexpr int G = (NT + 3) / 4;
+    Cx<R> pre[G];
+    uint32_t left = phases;
+    auto fetch = [&] {
+        if (!left) return;
+        left--;
+#pragma unroll
+        for (int g = 0; g < G; g++) pre[g] = pt[16 * g + ((threadIdx.x >> (4 * g)) & 15u)];
+        pt += 16 * G;
+    };
+    fetch();
+    uint32_t cw = codes[0], next = codes[1], n = 0;
+    for (;;) {
+        const uint32_t code = cw & 0xFFu;
+        if (code == SC_END) return;
+        cw >>= 8;
+        if ((++n & 3u) == 0) {
+            cw = next;
+            next = codes[(n >> 2) + 1];
+        }
+        switch (code) {
+#define RO(D) \
+    case D: rotate<D>(v, cf[0].re, cf[0].im); cf++; break;
+            RO(1) RO(2) RO(3) RO(4) RO(5) RO(6) RO(7) RO(8) RO(9) RO(10) RO(11) RO(12) RO(13) RO(14) RO(15)
+#undef RO
+        case SC_DIAG:
+#pragma unroll
+            for (int s = 0; s < 16; s++) v[s] = cmul(cf[s], v[s]);
+            cf += 16;
+            break;
+        case SC_LAYER:
+            rotate<1>(v, cf[0].re, cf[0].im);
+            rotate<2>(v, cf[1].re, cf[1].im);
+            rotate<4>(v, cf[2].re, cf[2].im);
+            rotate<8>(v, cf[3].re, cf[3].im);
+#pragma unroll
+            for (int s = 0; s < 16; s++) v[s] = cmul(cf[4 + s], v[s]);
+            cf += 20;
+            break;
+        default: {
+            Cx<R> h = *tile_phase++;
+#pragma unroll
+            for (int g = 0; g < G; g++) h = cmul(pre[g], h);
+            fetch();
+            switch (code - SC_PHASE) {
+#define PH(M) \
+    case M: phase<M, 0>(v, h); break; \
+    case (M) + 16: phase<M, 1>(v, h); break;
+                PH(1) PH(2) PH(3) PH(4) PH(5) PH(6) PH(7) PH(8) PH(9) PH(10) PH(11) PH(12) PH(13) PH(14) PH(15)
+#undef PH
+            default: __builtin_unreachable();
+            }
+            break;
+        }
+        }
+    }
+}
+
+// All ones if bit i of x is set.
+__device__ __forceinline__ uint32_t bit_mask(uint32_t x, int i) { return (uint32_t)((int32_t)(x << (31 - i)) >> 31); }
+
+__device__ __forceinline__ uint64_t bit_select(uint32_t x, int i, uint64_t y)
+{
+    const uint32_t m = bit_mask(x, i);
+    return ((uint64_t)(m & (uint32_t)(y >> 32)) << 32) | (m & (uint32_t)y);
+}
+
+constexpr uint32_t kTouchLines = 8;
+
+// A streamed step's scalar words and this thread's LDS offset in it, loaded
+// one step ahead.
+struct StreamStep {
+    uint32_t codes, phase, coef, phase_coef, lines;  // lines: 64-byte lines of the step's coefficients
+    uint32_t r[4], w[4], flip;  // LDS byte offsets of the register bits as read and as written
+    uint32_t base;
+};
+
+template <int TB, int NB>
+__device__ __forceinline__ StreamStep load_stream_step(const MicroStep* __restrict__ ms, uint32_t tid)
+{
+    const uint32_t* __restrict__ w = reinterpret_cast<const uint32_t*>(ms);
+    StreamStep st;
+    st.codes = w[1];
+    st.phase = w[2];
+    st.phase_coef = w[25];
+    st.coef = w[3];
+    st.lines = w[0] >> 16;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        st.r[k] = w[4 + k];
+        st.w[k] = w[8 + k];
+    }
+    st.flip = w[12];
+    st.base = 0;
+#pragma unroll
+    for (int i = 0; i < TB - NB; i++) st.base ^= bit_mask(tid, i) & w[13 + i];
+    return st;
+}
+
+// Waves per SIMD: what the LDS tiles allow.
+template <typename R, int TB>
+constexpr int kStreamWavesPerEU = kLdsWavesPerSimd<R, TB, 4> > 4 ? 4 : kLdsWavesPerSimd<R, TB, 4>;
+
+template <typename R, int TB>
+__global__ __launch_bounds__(1 << (TB - 4)) __attribute__((amdgpu_waves_per_eu(kStreamWavesPerEU<R, TB>)))
+void k_stream(const Cx<R>* state, PassArgs pa, const MicroStep* __restrict__ micro,
+              const uint32_t* __restrict__ codes, const Phase* __restrict__ phases,
+              const Cx<R>* __restrict__ coef, Cx<R>* out, const ScatterArgs* __restrict__ sa)
+{
+    constexpr int NB = 4, N = 1 << NB, NT = 1 << (TB - NB);
+    __shared__ Cx<R> tile[1 << TB];
+    __shared__ Cx<R> tile_phase[kTilePhases];
+    const uint32_t tid = threadIdx.x;
+    const uint64_t blk = blockIdx.x, base = rest_base(pa, blk);
+    const MicroStep* __restrict__ ms = micro + pa.micro_begin;
+    Cx<R> v[N];
+    {
+        // the first step's amplitudes straight into its registers, or the
+        // tile in load order
+        uint64_t tb = base, g[NB];
+        if (pa.fuse_first) {
+#pragma unroll
+            for (int i = 0; i < TB - NB; i++) tb ^= bit_select(tid, i, pa.first_g[i]);
+#pragma unroll
+            for (int k = 0; k < NB; k++) g[k] = pa.first_g[12 + k];
+        } else {
+#pragma unroll
+            for (int b = 0; b < TB - NB; b++) tb ^= bit_select(tid, b, 1ull << pa.load_pos[b]);
+#pragma unroll
+            for (int k = 0; k < NB; k++) g[k] = 1ull << pa.load_pos[TB - NB + k];
+        }
+        auto offset = [&](int s) {
+            uint64_t off = tb;
+#pragma unroll
+            for (int k = 0; k < NB; k++)
+                if ((s >> k) & 1) off ^= g[k];
+            return off;
+        };
+        if (pa.synth_basis) {
+#pragma unroll
+            for (int s = 0; s < N; s++) v[s] = synth_amp<R>(pa, offset(s));
+        } else if (pa.zero_mask) {
+#pragma unroll
+            for (int s = 0; s < N; s++) v[s] = masked_load(state, pa, offset(s));
+        } else {
+#pragma unroll
+            for (int s = 0; s < N; s++) v[s] = state[offset(s)];
+        }
+    }
+    // the tile's factors of the pass's phases, one thread each, while the
+    // amplitudes come in
+    for (uint32_t p = tid; p < pa.phase_count; p += NT) {
+        const Phase* __restrict__ ph = phases + pa.phase_begin + p;
+        Cx<R> h{(R)1, (R)0};
+        const uint32_t groups = ph->groups;
+        for (uint32_t g = 0; g < groups; g++) {
+            const uint32_t w = ph->pos[g];
+            uint32_t e = 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) e |= (uint32_t)((base >> ((w >> (8 * i)) & 63u)) & 1ull) << i;
+            h = cmul(coef[ph->coef + 16 * g + e], h);
+        }
+        tile_phase[p] = h;
+    }
+    if (!pa.fuse_first) {
+        const uint32_t tsw = swz<R>(tid) * (uint32_t)sizeof(Cx<R>);
+#pragma unroll
+        for (int i = 0; i < N; i++) lds_at(tile, tsw ^ (swz<R>((uint32_t)i * NT) * (uint32_t)sizeof(Cx<R>))) = v[i];
+    }
+    if (!pa.fuse_first || pa.phase_count) __syncthreads();
+    StreamStep st;
+    if (pa.micro_count) st = load_stream_step<TB, NB>(ms, tid);
+    for (uint32_t mi = 0; mi < pa.micro_count; mi++) {
+        // the lines of the step's coefficients, fetched into the scalar cache
+        // under the LDS reads
+        uint32_t touched = 0;
+        {
+            const char* __restrict__ p = reinterpret_cast<const char*>(coef + st.coef);
+#pragma unroll
+            for (uint32_t i = 0; i < kTouchLines; i++)
+                touched ^= *reinterpret_cast<const uint32_t*>(p + 64 * (i < st.lines ? i : st.lines - 1));
+        }
+        if (mi || !pa.fuse_first) {
+#pragma unroll
+            for (int s = 0; s < N; s++) v[s] = lds_at(tile, st.base ^ reg_offset<NB>(s, st.r));
+        }
+        asm volatile("" ::"s"(touched));
+        const uint32_t next_phase = mi + 1 < pa.micro_count ? reinterpret_cast<const uint32_t*>(ms + mi + 1)[2] : pa.phase_count;
+        stream_ops<R, TB - NB>(v, codes + st.codes, coef + st.coef, coef + st.phase_coef, tile_phase + st.phase,
+                               next_phase - st.phase);
+        if (mi + 1 == pa.micro_count) {
+            if (pa.fuse_last) break;
+        }
+        const uint32_t wb = st.base ^ st.flip;
+        uint32_t w[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) w[k] = st.w[k];
+        // the next step's words come in under the LDS writes
+        if (mi + 1 < pa.micro_count) st = load_stream_step<TB, NB>(ms + mi + 1, tid);
+#pragma unroll
+        for (int s = 0; s < N; s++) lds_at(tile, wb ^ reg_offset<NB>(s, w)) = v[s];
+        __syncthreads();
+    }
+    uint64_t tb = pa.scatter ? out_base(pa, blk, sa + pa.scatter_idx) : base, g[NB];
+    if (pa.fuse_last) {
+        // in place, a one-step pass stores where other threads of the tile
+        // load: every load has completed once all threads pass this barrier
+        if (pa.micro_count == 1) __syncthreads();
+        tb ^= pa.last_xor;
+#pragma unroll
+        for (int i = 0; i < TB - NB; i++) tb ^= bit_select(tid, i, pa.last_g[i]);
+#pragma unroll
+        for (int k = 0; k < NB; k++) g[k] = pa.last_g[12 + k];
+    } else {
+        uint32_t rbase = 0, r[4];
+#pragma unroll
+        for (int b = 0; b < TB - NB; b++) {
+            rbase ^= bit_mask(tid, b) & pa.store_byte[b];
+            tb ^= bit_select(tid, b, pa.scatter ? sa[pa.scatter_idx].out_tile[b] : 1ull << pa.store_pos[b]);
+        }
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            r[k] = pa.store_byte[TB - NB + k];
+            g[k] = pa.scatter ? sa[pa.scatter_idx].out_tile[TB - NB + k] : 1ull << pa.store_pos[TB - NB + k];
+        }
+#pragma unroll
+        for (int s = 0; s < N; s++) v[s] = lds_at(tile, rbase ^ reg_offset<NB>(s, r));
+    }
+#pragma unroll
+    for (int s = 0; s < N; s++) {
+        uint64_t off = tb;
+#pragma unroll
+        for (int k = 0; k < NB; k++)
+            if ((s >> k) & 1) off ^= g[k];
+        out[off] = v[s];
+    }
+}
+
+template <typename R, int TB>
+int stream_t(void* state, const PassArgs& pa, const DevPlan& dp, hipStream_t s)
+{
+    hipLaunchKernelGGL((k_stream<R, TB>), dim3(1u << pa.nrest), dim3(1 << (TB - 4)), 0, s, (const Cx<R>*)state, pa,
+                       dp.micro, dp.raw, dp.phases, (const Cx<R>*)dp.coef, (Cx<R>*)(pa.scatter ? dp.dst : state), dp.scatter);
+    return (int)hipGetLastError();
+}
+
+template <typename R>
+int stream_r(int tile_bits, void* state, const PassArgs& pa, const DevPlan& dp, hipStream_t s)
+{
+    if (pa.micro_bits != 4 || (pa.scatter && (!dp.dst || !dp.scatter)) || pa.phase_count > kTilePhases ||
+        (pa.phase_count && !dp.phases))
+        return (int)hipErrorInvalidValue;
+    // the planner streams only plans whose tile size it chose: 12 qubits, or 13
+    // for complex64 plans of light passes, whose permutations stay off k_stream
+    if (tile_bits != 12) return (int)hipErrorInvalidValue;
+    return stream_t<R, 12>(state, pa, dp, s);
 }
 
 // ---- many circuits in one persistent launch ---------------------------------

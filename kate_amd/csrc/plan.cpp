@@ -28,8 +28,12 @@ inline int popc(uint64_t x) { return __builtin_popcountll(x); }
 // Which gates of `masks` (in order) run when only the qubits in `set` are
 // available: a gate runs if its qubits are in `set` and no earlier gate
 // sharing a qubit with it was left out.  Gates with ok[i] == 0 never run.
+// A gate with any[i] needs only one of its qubits in `set` (`any` may be
+// empty: none).
+inline bool held_in(uint64_t m, uint64_t set, bool any) { return any ? (m & set) != 0 : (m & ~set) == 0; }
+
 int sweep(const std::vector<uint64_t>& masks, const std::vector<uint8_t>& ok, uint64_t set, uint64_t universe,
-          std::vector<int>* frontier, std::vector<int>* accepted)
+          std::vector<int>* frontier, std::vector<int>* accepted, const std::vector<uint8_t>& any = {})
 {
     uint64_t blocked = 0;
     int count = 0;
@@ -37,7 +41,7 @@ int sweep(const std::vector<uint64_t>& masks, const std::vector<uint8_t>& ok, ui
         const uint64_t m = masks[i];
         if (m & blocked) {
             blocked |= m;
-        } else if (ok[i] && (m & ~set) == 0) {
+        } else if (ok[i] && held_in(m, set, !any.empty() && any[i])) {
             count++;
             if (accepted) accepted->push_back((int)i);
         } else {
@@ -54,7 +58,8 @@ int sweep(const std::vector<uint64_t>& masks, const std::vector<uint8_t>& ok, ui
 // register op, any other is applied to the tile layout after the step; a
 // gate after a layout CNOT on one of its qubits waits for the next step.
 int sweep_micro(const std::vector<uint64_t>& masks, const std::vector<uint8_t>& ok, const std::vector<uint8_t>& lazy,
-                uint64_t set, std::vector<int>* frontier, std::vector<int>* reg, std::vector<int>* late)
+                uint64_t set, std::vector<int>* frontier, std::vector<int>* reg, std::vector<int>* late,
+                const std::vector<uint8_t>& any = {})
 {
     uint64_t blocked = 0, pending = 0;
     int count = 0;
@@ -70,7 +75,7 @@ int sweep_micro(const std::vector<uint64_t>& masks, const std::vector<uint8_t>& 
                 pending |= m;
                 if (late) late->push_back((int)i);
             }
-        } else if (ok[i] && (m & ~set) == 0 && !(m & pending)) {
+        } else if (ok[i] && held_in(m, set, !any.empty() && any[i]) && !(m & pending)) {
             count++;
             if (reg) reg->push_back((int)i);
         } else {
@@ -82,26 +87,31 @@ int sweep_micro(const std::vector<uint64_t>& masks, const std::vector<uint8_t>& 
 }
 
 uint64_t choose_micro_set(const std::vector<uint64_t>& masks, const std::vector<uint8_t>& ok,
-                          const std::vector<uint8_t>& lazy, int width)
+                          const std::vector<uint8_t>& lazy, int width, const std::vector<uint8_t>& any = {})
 {
     uint64_t set = 0;
     for (;;) {
         std::vector<int> frontier;
-        const int now = sweep_micro(masks, ok, lazy, set, &frontier, nullptr, nullptr);
+        const int now = sweep_micro(masks, ok, lazy, set, &frontier, nullptr, nullptr, any);
         double best = 0;
         uint64_t best_new = 0;
         std::vector<uint64_t> tried;
-        for (int f : frontier) {
-            const uint64_t add = masks[(size_t)f] & ~set;
-            if (popc(set | add) > width) continue;
-            if (std::find(tried.begin(), tried.end(), add) != tried.end()) continue;
+        auto consider = [&](uint64_t add) {
+            if (popc(set | add) > width) return;
+            if (std::find(tried.begin(), tried.end(), add) != tried.end()) return;
             tried.push_back(add);
-            const int gain = sweep_micro(masks, ok, lazy, set | add, nullptr, nullptr, nullptr) - now;
+            const int gain = sweep_micro(masks, ok, lazy, set | add, nullptr, nullptr, nullptr, any) - now;
             const double score = (double)gain / popc(add);
             if (score > best) {
                 best = score;
                 best_new = add;
             }
+        };
+        for (int f : frontier) {
+            const uint64_t add = masks[(size_t)f] & ~set;
+            if (!any.empty() && any[(size_t)f])
+                for (uint64_t m = add; m; m &= m - 1) consider(m & (~m + 1));
+            else consider(add);
         }
         if (!best_new) return set;
         set |= best_new;
@@ -112,26 +122,31 @@ uint64_t choose_micro_set(const std::vector<uint64_t>& masks, const std::vector<
 // qubits of the ready gate that makes the most gates runnable per added
 // qubit (earliest gate on ties).
 uint64_t choose_set(const std::vector<uint64_t>& masks, const std::vector<uint8_t>& ok, int capacity, uint64_t start,
-                    uint64_t universe)
+                    uint64_t universe, const std::vector<uint8_t>& any = {})
 {
     uint64_t set = start;
     for (;;) {
         std::vector<int> frontier;
-        const int now = sweep(masks, ok, set, universe, &frontier, nullptr);
+        const int now = sweep(masks, ok, set, universe, &frontier, nullptr, any);
         double best = 0;
         uint64_t best_new = 0;
         std::vector<uint64_t> tried;
-        for (int f : frontier) {
-            const uint64_t add = masks[(size_t)f] & ~set;
-            if (popc(set | add) > capacity) continue;
-            if (std::find(tried.begin(), tried.end(), add) != tried.end()) continue;
+        auto consider = [&](uint64_t add) {
+            if (popc(set | add) > capacity) return;
+            if (std::find(tried.begin(), tried.end(), add) != tried.end()) return;
             tried.push_back(add);
-            const int gain = sweep(masks, ok, set | add, universe, nullptr, nullptr) - now;
+            const int gain = sweep(masks, ok, set | add, universe, nullptr, nullptr, any) - now;
             const double score = (double)gain / popc(add);
             if (score > best) {
                 best = score;
                 best_new = add;
             }
+        };
+        for (int f : frontier) {
+            const uint64_t add = masks[(size_t)f] & ~set;
+            if (!any.empty() && any[(size_t)f])
+                for (uint64_t m = add; m; m &= m - 1) consider(m & (~m + 1));
+            else consider(add);
         }
         if (!best_new) return set;
         set |= best_new;
@@ -303,6 +318,8 @@ struct Builder {
     Plan& plan;
     uint64_t zero = ~0ull;  // qubits still exactly |0> in a run from |0...0>
     bool remapped = false;  // a remap pass was planned: support no longer tracked
+    uint32_t phase_begin = 0;  // first phase of the pass being packed
+    bool phases = false;    // CRk gates need only one of their qubits in the tile and in registers
 
     // Support update for one gate (sound: a qubit stays in `zero` only if
     // every amplitude with that bit set is still exactly zero).
@@ -404,6 +421,7 @@ struct Builder {
         pa.fuse_first = pa.fuse_last = 0;
         std::fill(pa.first_g, pa.first_g + 16, 0ull);
         std::fill(pa.last_g, pa.last_g + 16, 0ull);
+        pa.last_xor = 0;
         if (!opt.direct || pa.micro_count == 0) return;
         const int t = plan.tile_bits, nb = opt.micro_bits, nt = t - nb;
         const int low = std::min(opt.low_qubits, nt);
@@ -463,13 +481,22 @@ struct Builder {
             };
             std::fill(g, g + 16, 0ull);
             for (int i = 0; i < nt; i++) g[i] = offset(tile_index(l.tcols[i]), pa.store_pos);
-            for (int k = 0; k < nb; k++) g[12 + k] = offset(tile_index(l.pcols[k]), pa.store_pos);
+            if (pa.stream) {
+                // register s holds the amplitude at LDS index wcol(s)
+                for (int k = 0; k < nb; k++) g[12 + k] = offset(tile_index(out_cols[k]), pa.store_pos);
+            } else {
+                for (int k = 0; k < nb; k++) g[12 + k] = offset(tile_index(l.pcols[k]), pa.store_pos);
+            }
             if (coalesced(g)) {
                 std::copy(g, g + 16, pa.last_g);
+                if (pa.stream) pa.last_xor = offset(tile_index(out_cols[4]), pa.store_pos);
                 pa.fuse_last = 1;
             }
         }
     }
+
+    uint32_t out_cols[5] = {0, 0, 0, 0, 0};  // of the last streamed step packed: LDS columns of its register bits
+                                             // as written, and of its flip
 
     int micro_bit(int tile_bit, const uint8_t* bits) const
     {
@@ -856,8 +883,346 @@ struct Builder {
         plan.ops.push_back(op);
     }
 
-    // Packs the gates of one pass (`gl`, program order) into micro-steps.
+    // Euler form of a 2x2 unitary, as euler_form, but defined for every
+    // unitary: the phases come from its larger entries, and an entry below
+    // rounding (4e-16) counts as zero.  Fails if u is not unitary to 1e-14.
+    static bool euler_any(const double* u, double& x, double& y, std::complex<double> (&p)[2],
+                          std::complex<double>& q)
+    {
+        using cd = std::complex<double>;
+        const cd u00(u[0], u[1]), u01(u[2], u[3]), u10(u[4], u[5]), u11(u[6], u[7]), I(0.0, 1.0);
+        x = std::abs(u00);
+        y = std::abs(u10);
+        if (x > 4e-16 && y > 4e-16) {
+            p[0] = u00 / x;
+            p[1] = I * u10 / y;
+            q = x >= y ? u11 / (std::abs(u11) * p[1]) : I * u01 / (std::abs(u01) * p[0]);
+            if (std::abs(q + 1.0) <= 2e-15) {  // a negative rotation, no right diagonal
+                y = -y;
+                p[1] = -p[1];
+                q = 1.0;
+            } else if (std::abs(q - 1.0) <= 2e-15) {
+                q = 1.0;
+            }
+        } else if (x > y) {  // diagonal
+            p[0] = u00 / x;
+            p[1] = u11 / std::abs(u11);
+            q = 1.0;
+            y = 0.0;
+        } else if (y > 0) {  // exchange
+            p[0] = I * u01 / std::abs(u01);
+            p[1] = I * u10 / y;
+            q = 1.0;
+            x = 0.0;
+        } else {
+            return false;
+        }
+        const cd r00 = p[0] * x, r01 = -I * p[0] * y * q, r10 = -I * p[1] * y, r11 = p[1] * x * q;
+        return std::max(std::max(std::abs(r00 - u00), std::abs(r01 - u01)),
+                        std::max(std::abs(r10 - u10), std::abs(r11 - u11))) <= 1e-14;
+    }
+
+    // One register step as a stream of rotations and diagonals.  Register s
+    // of a thread holds the amplitude of register-bit values A s ^ f (A
+    // invertible over GF(2)): a CNOT only changes A and f, a rotation of
+    // qubit bit j runs along the register direction A^-1 e_j, and the step's
+    // write addresses undo A and f.  Diagonal factors collect in `d` (by
+    // register) and are applied before the next rotation that does not
+    // commute with them.
+    struct Stream {
+        int col[4] = {1, 2, 4, 8};  // A's columns
+        int f = 0;
+        std::complex<double> d[16];
+        // pending phases of register bit j with a thread-index bit or a state
+        // offset bit outside the tile
+        struct Pending {
+            bool thread;
+            int bit;
+            std::complex<double> f;
+        };
+        std::vector<Pending> phase[4];
+        std::vector<uint8_t> codes;
+        std::vector<double> coef;
+        std::vector<double> thread_coef, tile_coef;  // tables of the SC_PHASE ops
+        std::vector<Phase> phases;                   // (coef: offset into tile_coef)
+        int thread_bits = 0;
+        Stream() { std::fill(d, d + 16, std::complex<double>(1.0)); }
+        void emit_phase(int j)
+        {
+            std::vector<Pending>& ph = phase[j];
+            if (ph.empty()) return;
+            int m = 0;
+            for (int k = 0; k < 4; k++)
+                if ((col[k] >> j) & 1) m |= 1 << k;
+            codes.push_back((uint8_t)(SC_PHASE + m + 16 * ((f >> j) & 1)));
+            // one factor per bit (gates on the same pair multiply)
+            std::vector<Pending> one;
+            for (const Pending& p : ph) {
+                auto it = std::find_if(one.begin(), one.end(),
+                                       [&](const Pending& o) { return o.thread == p.thread && o.bit == p.bit; });
+                if (it == one.end()) one.push_back(p);
+                else it->f *= p.f;
+            }
+            auto table = [](std::vector<double>& out, const std::vector<std::complex<double>>& fs) {
+                for (int e = 0; e < 16; e++) {
+                    std::complex<double> t = 1.0;
+                    for (size_t i = 0; i < fs.size(); i++)
+                        if ((e >> i) & 1) t *= fs[i];
+                    out.push_back(t.real());
+                    out.push_back(t.imag());
+                }
+            };
+            for (int g = 0; 4 * g < thread_bits; g++) {
+                std::vector<std::complex<double>> fs(4, 1.0);
+                for (const Pending& p : one)
+                    if (p.thread && p.bit / 4 == g) fs[(size_t)(p.bit % 4)] = p.f;
+                table(thread_coef, fs);
+            }
+            std::vector<Pending> rest;
+            for (const Pending& p : one)
+                if (!p.thread) rest.push_back(p);
+            kate::Phase tile{};
+            tile.groups = (uint32_t)((rest.size() + 3) / 4);
+            tile.coef = (uint32_t)(tile_coef.size() / 2);
+            for (uint32_t g = 0; g < tile.groups; g++) {
+                std::vector<std::complex<double>> fs;
+                for (size_t i = 0; i < 4; i++) {
+                    const bool have = 4 * g + i < rest.size();
+                    tile.pos[g] |= (have ? (uint32_t)rest[4 * g + i].bit : 63u) << (8 * i);
+                    if (have) fs.push_back(rest[4 * g + i].f);
+                }
+                table(tile_coef, fs);
+            }
+            phases.push_back(tile);
+            ph.clear();
+        }
+        int value(int s) const
+        {
+            int v = f;
+            for (int k = 0; k < 4; k++)
+                if ((s >> k) & 1) v ^= col[k];
+            return v;
+        }
+        int direction(int bits) const  // the register direction that changes exactly these bits
+        {
+            for (int s = 1; s < 16; s++)
+                if ((value(s) ^ f) == bits) return s;
+            return 0;
+        }
+        void emit_diag()
+        {
+            bool one = true;
+            for (const auto& v : d) one = one && v == 1.0;
+            if (one) return;
+            codes.push_back(SC_DIAG);
+            for (auto& v : d) {
+                coef.push_back(v.real());
+                coef.push_back(v.imag());
+                v = 1.0;
+            }
+        }
+        bool commutes(int dir) const
+        {
+            for (int s = 0; s < 16; s++)
+                if (d[s] != d[s ^ dir]) return false;
+            return true;
+        }
+        void cnot(int target, int control)
+        {
+            auto c = [&](int v) { return ((v >> control) & 1) ? v ^ (1 << target) : v; };
+            for (int& v : col) v = c(v);
+            f = c(f);
+        }
+    };
+
+    // The held 1-qubit gates of the register bits in `mask`, together: their
+    // right diagonals, their rotations (scaled by their larger entry, see
+    // factor_ekron: the smaller quotient is applied, outputs exchanged through
+    // f), their left diagonals.
+    bool stream_flush(Stream& st, Held* held, int mask)
+    {
+        double xs[4], ys[4];
+        std::complex<double> ps[4][2], qs[4];
+        for (int j = 0; j < 4; j++) {
+            if (!((mask >> j) & 1) || !held[j].count) continue;
+            if (!euler_any(held[j].m, xs[j], ys[j], ps[j], qs[j])) return false;
+        }
+        for (int j = 0; j < 4; j++) {
+            if (!((mask >> j) & 1) || !held[j].count || qs[j] == 1.0) continue;
+            for (int s = 0; s < 16; s++)
+                if ((st.value(s) >> j) & 1) st.d[s] *= qs[j];
+        }
+        // the order of the rotations is free: one whose lowest direction bit no
+        // other remaining one changes goes first, so that its scale commutes
+        // with the rest
+        int left = 0;
+        for (int j = 0; j < 4; j++)
+            if (((mask >> j) & 1) && held[j].count) left |= 1 << j;
+        while (left) {
+            int j = __builtin_ctz((unsigned)left);
+            for (int c = 0; c < 4; c++) {
+                if (!((left >> c) & 1)) continue;
+                const int dc = st.direction(1 << c), low = dc & -dc;
+                bool alone = true;
+                for (int o = 0; o < 4; o++)
+                    if (o != c && ((left >> o) & 1) && (st.direction(1 << o) & low)) alone = false;
+                if (alone) {
+                    j = c;
+                    break;
+                }
+            }
+            left &= ~(1 << j);
+            const double x = xs[j], y = ys[j];
+            const int dir = st.direction(1 << j), low = dir & -dir;
+            if (y != 0.0) st.emit_phase(j);
+            std::complex<double> scale = x;
+            double t = 0.0;
+            if (std::abs(x) >= std::abs(y)) {
+                t = y / x;
+            } else {
+                t = -x / y;
+                scale = std::complex<double>(0.0, -y);
+                st.f ^= 1 << j;
+            }
+            if (t != 0.0) {
+                if (!st.commutes(dir)) st.emit_diag();
+                st.codes.push_back((uint8_t)dir);
+                st.coef.push_back(t);
+                st.coef.push_back(t / (1.0 + t * t));
+            }
+            for (int s = 0; s < 16; s++) {
+                st.d[s] *= scale * ps[j][(st.value(s) >> j) & 1];
+                if (t != 0.0 && (s & low)) st.d[s] *= 1.0 + t * t;
+            }
+            held[j] = Held();
+        }
+        return true;
+    }
+
+    // Gates a streamed pass can run.
+    bool streamable(const PlanGate& g) const
+    {
+        return g.id == 2 || g.id == 3 || g.id == 4 || (g.id == 0 && g.k == 1);
+    }
+
+    // The gates `acc` of a register step as a stream in `ms`.
+    // lane[i] is the tile bit of thread-index bit i.
+    bool stream_step(const std::vector<int>& rem, const std::vector<int>& acc, const int* tile_of,
+                     const std::vector<int>& lane, MicroStep& ms)
+    {
+        Stream st;
+        st.thread_bits = (int)lane.size();
+        Held held[4];
+        for (int a : acc) {
+            const PlanGate& g = prog.gates[(size_t)rem[(size_t)a]];
+            int b[16], touched = 0, outside = -1;
+            for (int i = 0; i < g.k; i++) {
+                b[i] = micro_bit(tile_of[g.q[i]], ms.bits);
+                if (b[i] >= 0) touched |= 1 << b[i];
+                else outside = g.q[i];
+            }
+            if (g.k == 1) {
+                hold(held[b[0]], g);
+                continue;
+            }
+            if (!stream_flush(st, held, touched)) return false;
+            if (g.id == 3) {
+                st.emit_phase(b[0]);
+                st.cnot(b[0], b[1]);
+            } else if (outside >= 0) {  // CRk with one qubit in registers
+                const double ang = ((double)2 * 3.1415926535897932384626433) / (double)(1ull << g.optarg);
+                const int tb = tile_of[outside];
+                Stream::Pending ph{tb >= 0, outside, {std::cos(ang), std::sin(ang)}};
+                if (tb >= 0) ph.bit = (int)(std::find(lane.begin(), lane.end(), tb) - lane.begin());
+                st.phase[__builtin_ctz((unsigned)touched)].push_back(ph);
+            } else {  // CRk
+                const double ang = ((double)2 * 3.1415926535897932384626433) / (double)(1ull << g.optarg);
+                const std::complex<double> ph(std::cos(ang), std::sin(ang));
+                for (int s = 0; s < 16; s++)
+                    if ((st.value(s) & touched) == touched) st.d[s] *= ph;
+            }
+        }
+        if (!stream_flush(st, held, 15)) return false;
+        for (int j = 0; j < 4; j++) st.emit_phase(j);
+        st.emit_diag();
+        // rotations of all four register bits and a diagonal: one op
+        for (size_t i = 0; i + 4 < st.codes.size(); i++)
+            if (st.codes[i] == 1 && st.codes[i + 1] == 2 && st.codes[i + 2] == 4 && st.codes[i + 3] == 8 &&
+                st.codes[i + 4] == SC_DIAG) {
+                st.codes.erase(st.codes.begin() + (long)i, st.codes.begin() + (long)i + 4);
+                st.codes[i] = SC_LAYER;
+            }
+        ms.coef = add_coef(st.coef.data(), st.coef.size() / 2);
+        ms.op_count = (uint32_t)(plan.phases.size() - phase_begin);
+        ms.phase_coef = add_coef(st.thread_coef.data(), st.thread_coef.size() / 2);
+        const uint32_t tile_coef = add_coef(st.tile_coef.data(), st.tile_coef.size() / 2);
+        for (Phase p : st.phases) {
+            p.coef += tile_coef;
+            plan.phases.push_back(p);
+        }
+        const size_t bytes = st.coef.size() * (size_t)opt.amp_bytes / 2;
+        ms.op0_code = (uint16_t)std::min<size_t>(std::max<size_t>((bytes + 63) / 64, 1), 0xFFFF);
+        if (!bytes) ms.coef = 0;  // an empty stream: its one line is the pool's first
+        ms.op_begin = (uint32_t)plan.raw.size();
+        // (a word of padding: the kernel loads one word ahead)
+        plan.raw.resize(plan.raw.size() + st.codes.size() / 4 + 2, 0u);
+        for (size_t i = 0; i < st.codes.size(); i++)
+            plan.raw[ms.op_begin + i / 4] |= (uint32_t)st.codes[i] << (8 * (i % 4));
+        auto lds_col = [&](int v) {
+            uint32_t c = 0;
+            for (int k = 0; k < 4; k++)
+                if ((v >> k) & 1) c ^= ms.cols[ms.bits[k]];
+            return c;
+        };
+        for (int k = 0; k < 4; k++) out_cols[k] = lds_col(st.col[k]);
+        out_cols[4] = lds_col(st.f);
+        for (int k = 0; k < 4; k++) ms.wbyte[k] = lds_bytes(out_cols[k]);
+        ms.wflip = lds_bytes(out_cols[4]);
+        return true;
+    }
+
+    // Packs the gates of one pass (`gl`, program order) into micro-steps:
+    // streamed if they all allow it and the light kernel does not, else as
+    // register ops and wide steps.  Light passes (30-qubit layered circuit,
+    // complex128: 6.9 ms a sweep pass, 13.0 ms a pass that mixes CNOTs and
+    // rotations; 28 qubits complex64, 13-qubit tiles: 1.2 and 2.2-2.6 ms) run
+    // 5 % slower streamed (7.4, 13.3; 1.2, 2.3-2.7); passes of CRk gates run
+    // several times faster, most of all because far fewer remain (25-qubit
+    // QFT: 14 passes, 5.05 ms; streamed with phases 3 passes, 1.33 ms).
     std::string pack_micro(const std::vector<int>& gl, const int* tile_of, PassArgs& pa)
+    {
+        if (opt.stream && opt.micro_bits == 4) {
+            bool all = true;
+            for (int g : gl) all = all && streamable(prog.gates[(size_t)g]);
+            if (all) {
+                const size_t nm = plan.micro.size(), no = plan.ops.size(), nc = plan.coef.size(), nr = plan.raw.size(),
+                             np = plan.phases.size();
+                auto undo = [&] {
+                    plan.phases.resize(np);
+                    plan.micro.resize(nm);
+                    plan.ops.resize(no);
+                    plan.coef.resize(nc);
+                    plan.raw.resize(nr);
+                };
+                // passes of the light set stay on the light kernel
+                std::string e = phases ? "phases" : pack_micro_as(gl, tile_of, pa);
+                if (e.empty() && pa.light) return "";
+                undo();
+                pa.stream = 1;
+                phase_begin = pa.phase_begin = (uint32_t)np;
+                e = pack_micro_as(gl, tile_of, pa);
+                pa.phase_count = (uint32_t)(plan.phases.size() - np);
+                if (pa.phase_count > kTilePhases) e = "not streamable";
+                if (e != "not streamable" || phases) return e;
+                undo();
+                pa.stream = 0;
+                pa.phase_count = 0;
+            }
+        }
+        return pack_micro_as(gl, tile_of, pa);
+    }
+
+    std::string pack_micro_as(const std::vector<int>& gl, const int* tile_of, PassArgs& pa)
     {
         const int t = plan.tile_bits;
         const int nb = opt.micro_bits;
@@ -874,12 +1239,14 @@ struct Builder {
         };
         while (!rem.empty()) {
             std::vector<uint64_t> tm(rem.size());
-            std::vector<uint8_t> ok(rem.size()), lazy(rem.size());
+            std::vector<uint8_t> ok(rem.size()), lazy(rem.size()), any(phases ? rem.size() : 0, 0);
             for (size_t i = 0; i < rem.size(); i++) {
                 const PlanGate& g = prog.gates[(size_t)rem[i]];
                 uint64_t m = 0;
-                for (int j = 0; j < g.k; j++) m |= 1ull << tile_of[g.q[j]];
+                for (int j = 0; j < g.k; j++)
+                    if (tile_of[g.q[j]] >= 0) m |= 1ull << tile_of[g.q[j]];
                 tm[i] = m;
+                if (phases) any[i] = g.id == 4;
                 ok[i] = g.k <= nb && !(g.id == 0 && opt.mfma && g.k == 4);
                 lazy[i] = g.id == 3;
             }
@@ -922,9 +1289,9 @@ struct Builder {
                 rem.swap(next);
                 continue;
             }
-            const uint64_t set = choose_micro_set(tm, ok, lazy, nb);
+            const uint64_t set = choose_micro_set(tm, ok, lazy, nb, any);
             std::vector<int> acc, late;
-            sweep_micro(tm, ok, lazy, set, nullptr, &acc, &late);
+            sweep_micro(tm, ok, lazy, set, nullptr, &acc, &late, any);
             MicroStep ms{};
             std::copy(cols, cols + 16, ms.cols);
             if (acc.empty() && !late.empty()) {
@@ -985,7 +1352,16 @@ struct Builder {
             for (int b = 0; b < t; b++)
                 if ((full >> b) & 1ull) ms.bits[nb++] = (uint8_t)b;
             ms.op_begin = (uint32_t)plan.ops.size();
-            {
+            std::vector<int> rest;
+            for (int b = 0; b < t; b++) {
+                bool reg = false;
+                for (int k = 0; k < nb; k++) reg = reg || b == ms.bits[k];
+                if (!reg) rest.push_back(b);
+            }
+            const std::vector<int> order = lane_order(rest, ms.cols);
+            if (pa.stream) {
+                if (!stream_step(rem, acc, tile_of, order, ms)) return "not streamable";
+            } else {
                 // 1-qubit gates are held per micro bit and multiplied together
                 // (FP64, later gate on the left) until a gate on more qubits
                 // touches the bit; held gates of several bits go out as one op.
@@ -1006,19 +1382,12 @@ struct Builder {
                 }
                 flush(held, (1 << nb) - 1);
             }
-            ms.op_count = (uint32_t)(plan.ops.size() - ms.op_begin);
-            if (ms.op_count) {
+            if (!pa.stream) ms.op_count = (uint32_t)(plan.ops.size() - ms.op_begin);
+            if (!pa.stream && ms.op_count) {
                 ms.op0_code = plan.ops[ms.op_begin].code;
                 ms.coef = plan.ops[ms.op_begin].coef;
             }
             {
-                std::vector<int> rest;
-                for (int b = 0; b < t; b++) {
-                    bool reg = false;
-                    for (int k = 0; k < nb; k++) reg = reg || b == ms.bits[k];
-                    if (!reg) rest.push_back(b);
-                }
-                const std::vector<int> order = lane_order(rest, ms.cols);
                 int ti = 0;
                 for (int b : order)
                     if (ti < 12) ms.tcols[ti++] = ms.cols[b];
@@ -1050,13 +1419,13 @@ struct Builder {
         for (uint32_t m = pa.micro_begin; m < plan.micro.size(); m++) {
             const MicroStep& ms = plan.micro[m];
             if (ms.kind != SK_REG) pa.has_wide = 1;
-            for (uint32_t o = ms.op_begin; ms.kind == SK_REG && o < ms.op_begin + ms.op_count; o++)
+            for (uint32_t o = ms.op_begin; !pa.stream && ms.kind == SK_REG && o < ms.op_begin + ms.op_count; o++)
                 if (!light_op(plan.ops[o].code)) pa.light = 0;
         }
-        if (pa.has_wide) pa.light = 0;
+        if (pa.has_wide || pa.stream) pa.light = 0;
         // the light kernels take a step's lone Euler-form op on every
         // register bit in the scaled form
-        for (uint32_t m = pa.micro_begin; opt.factor && pa.light && m < plan.micro.size(); m++) {
+        for (uint32_t m = pa.micro_begin; opt.factor && pa.light && !pa.stream && m < plan.micro.size(); m++) {
             MicroStep& ms = plan.micro[m];
             if (ms.op_count != 1) continue;
             factor_ekron(plan.ops[ms.op_begin], ms.nbits);
@@ -1110,18 +1479,19 @@ struct Builder {
         std::vector<int> rem = seg;
         while (!rem.empty()) {
             std::vector<uint64_t> masks(rem.size());
-            std::vector<uint8_t> ok(rem.size(), 1);
+            std::vector<uint8_t> ok(rem.size(), 1), any(phases ? rem.size() : 0, 0);
             uint64_t universe = 0;
             for (size_t i = 0; i < rem.size(); i++) {
                 masks[i] = prog.gates[(size_t)rem[i]].mask;
                 universe |= masks[i];
+                if (phases) any[i] = prog.gates[(size_t)rem[i]].id == 4;
             }
             uint64_t start = low_mask;
             if (popc(low_mask | masks[0]) > t) start = pad_set(masks[0], std::min(t, popc(masks[0]) + low), n) & ~0ull;
             if (popc(start) > t) return "gate larger than the tile";
-            const uint64_t set = pad_set(choose_set(masks, ok, t, start, universe), t, n);
+            const uint64_t set = pad_set(choose_set(masks, ok, t, start, universe, any), t, n);
             std::vector<int> acc;
-            sweep(masks, ok, set, universe, nullptr, &acc);
+            sweep(masks, ok, set, universe, nullptr, &acc, any);
             if (acc.empty()) return "internal: empty pass";
             PassArgs pa{};
             pa.micro_bits = (uint8_t)opt.micro_bits;
@@ -1181,7 +1551,7 @@ struct Builder {
             pa.micro_begin = (uint32_t)plan.micro.size();
             pa.micro_count = 0;
             for (int b = 0; b < 16; b++) pa.store_cols[b] = (uint16_t)(1u << b);
-            fill_store_bytes(pa);
+                fill_store_bytes(pa);
             // a remap pass writes every tile (masked reads of the zero
             // qubits); the support is not tracked through it
             plan.pass_zero.push_back(remapped ? 0ull : zero);
@@ -1509,9 +1879,21 @@ static void make_relabel(Plan& plan)
             for (int p = 0; p < t; p++) sa.out_tile[p] = 1ull << Q[pa.store_pos[p]];
             for (int i = 0; i < pa.nrest; i++) sa.out_rest[i] = 1ull << Q[pa.rest_pos[i]];
             for (int i = 0; i < 16; i++) pa.last_g[i] = permute_bits(Q, pa.last_g[i]);
+            pa.last_xor = permute_bits(Q, pa.last_xor);
             pa.scatter = 1;
             pa.scatter_idx = (uint32_t)plan.scatter_args.size();
             plan.scatter_args.push_back(sa);
+        }
+        for (uint32_t i = 0; i < pa.phase_count; i++) {
+            Phase& ph = plan.phases[pa.phase_begin + i];
+            for (uint32_t g = 0; g < ph.groups; g++) {
+                uint32_t out = 0;
+                for (int j = 0; j < 4; j++) {
+                    const uint32_t q = (ph.pos[g] >> (8 * j)) & 255u;
+                    out |= (q < (uint32_t)n ? (uint32_t)P[q] : q) << (8 * j);
+                }
+                ph.pos[g] = out;
+            }
         }
         for (int b = 0; b < t; b++) pa.load_pos[b] = (uint8_t)P[pa.load_pos[b]];
         for (int i = 0; i < pa.nrest; i++) pa.rest_pos[i] = (uint8_t)P[pa.rest_pos[i]];
@@ -1602,7 +1984,7 @@ static double plan_cost(const Plan& p, int amp_bytes)
                 if ((p.pass_zero[i] >> pa.rest_pos[j]) & 1ull) f *= 0.5;
         // (a pass of the full op set is bound by its register steps; its
         // reads cost it what they cost in place)
-        const bool relabelled = p.relabel_begin >= 0 && (long)i >= p.relabel_begin && pa.light;
+        const bool relabelled = p.relabel_begin >= 0 && (long)i >= p.relabel_begin && (pa.light || pa.stream);
         c += f * (relabelled ? relabel_run_cost(run) : run_cost(run));
     }
     return c;
@@ -1704,7 +2086,22 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
     if (opt.amp_bytes != 16 && opt.amp_bytes != 8) return "amplitudes have 8 or 16 bytes";
     if (opt.micro_bits != 4 && (opt.mfma || opt.mfma_fuse || opt.mfma5)) return "matrix-core steps need 4-bit micro-steps";
     Builder b{prog, opt, plan};
+    if (opt.stream && opt.phases && opt.micro_bits == 4) {
+        // a program of gates that can all be streamed, CRk among them
+        bool all = true, crk = false;
+        for (const PlanGate& g : prog.gates) {
+            all = all && b.streamable(g);
+            crk = crk || g.id == 4;
+        }
+        b.phases = all && crk;
+    }
     b.zero = !opt.zero_start ? 0ull : plan.nq_int >= 64 ? ~0ull : ((1ull << plan.nq_int) - 1ull);
+    // a pass with phases outside its tile has no other form
+    auto without_phases = [&] {
+        PlanOptions o = opt;
+        o.phases = false;
+        return build_plan(prog, o, plan);
+    };
     std::vector<int> seg;
     size_t grp = 0;
     int first = 0;
@@ -1712,6 +2109,7 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
         if (prog.instr_kind[i] == 0) {
             if (!seg.empty()) {
                 std::string e = b.gate_passes(seg);
+                if (e == "not streamable") return without_phases();
                 if (!e.empty()) return e;
                 seg.clear();
             }
@@ -1726,6 +2124,7 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
     }
     if (!seg.empty()) {
         std::string e = b.gate_passes(seg);
+        if (e == "not streamable") return without_phases();
         if (!e.empty()) return e;
     }
     plan_trailing(plan);
@@ -1751,12 +2150,13 @@ std::string Plan::describe(bool verbose) const
             os << "]";
         }
         size_t nops = 0;
-        for (uint32_t m = 0; m < p.micro_count; m++) nops += micro[p.micro_begin + m].op_count;
+        for (uint32_t m = 0; !p.stream && m < p.micro_count; m++) nops += micro[p.micro_begin + m].op_count;
         os << " micro=" << p.micro_count << " ops=" << nops;
         if (p.fuse_first || p.fuse_last)
             os << " direct=" << (p.fuse_first ? "first" : "") << (p.fuse_first && p.fuse_last ? "," : "")
                << (p.fuse_last ? "last" : "");
         if (p.light && p.micro_count) os << " light";
+        if (p.stream && p.micro_count) os << " stream";
         if (p.scatter) os << ((long)i == scatter_pass ? " scatter" : " relabel");
         // state bits known zero at this pass's input in a run from |0...0>
         // (its loads skip those amplitudes)
@@ -1771,9 +2171,17 @@ std::string Plan::describe(bool verbose) const
             const int nb = ms.nbits;
             for (int b = 0; b < nb; b++) os << (b ? "," : "") << (int)ms.bits[b];
             os << "]";
-            for (uint32_t o = 0; o < ms.op_count; o++) {
+            for (uint32_t o = 0; !p.stream && o < ms.op_count; o++) {
                 const MicroOp& op = ops[ms.op_begin + o];
                 os << " " << okinds[op.code >> 8] << ":" << (op.code & 0xFF);
+            }
+            for (uint32_t o = 0; p.stream; o++) {
+                const int code = (int)(raw[ms.op_begin + o / 4] >> (8 * (o % 4))) & 255;
+                if (code == SC_END) break;
+                if (code == SC_DIAG) os << " diag";
+                else if (code == SC_LAYER) os << " layer";
+                else if (code >= SC_PHASE) os << " pphase:" << code - SC_PHASE;
+                else os << " rot:" << code;
             }
             if (ms.kind == SK_REG) {
                 os << " tcols=";

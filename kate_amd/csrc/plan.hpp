@@ -32,20 +32,59 @@ enum StepKind : uint8_t {
     SK_MFMA_BF16 = 3,  // the same with split-bf16 products (x = hi + lo, three products), FP32 accumulation
 };
 
+// Ops of a streamed step (PassArgs::stream): one byte each.
+enum StreamCode : uint8_t {
+    SC_END = 0,
+    // 1..15: rotation along direction d = code of the register index: every
+    // pair (s, s ^ d) becomes [[1, -it], [-it, 1]] of itself, its member with
+    // the lowest bit of d divided by 1 + t^2 (one in-place FMA per component);
+    // coefficients: one complex (t, t / (1 + t^2))
+    SC_DIAG = 16,   // every register times its entry of a 16-entry complex table
+    SC_LAYER = 17,  // rotations along 1, 2, 4, 8, then SC_DIAG, in one op
+    // 32 + m + 16 * p (m in 1..15): the registers s with parity(s & m) ^ p
+    // times a factor of the thread, the product of a table entry per four
+    // thread-index bits (MicroStep::phase_coef, 16 entries each) and of the
+    // tile's factor (Phase)
+    SC_PHASE = 32,
+};
+
+// The tile's factor of an SC_PHASE op: a product over groups of four state
+// offset bits of the tile's base, each group's bits (positions one a byte,
+// 63: none) picking one of 16 entries from `coef` on.
+constexpr uint32_t kTilePhases = 128;  // SC_PHASE ops per pass
+
+struct Phase {
+    uint32_t groups;
+    uint32_t coef;
+    uint32_t pos[10];
+};
+
 struct MicroOp {
     uint16_t code;
     uint16_t pad;
     uint32_t coef;  // complex-element offset into the coefficient pool
 };
 
-struct MicroStep {
+// The kernels read the fields up to tbyte as scalar words.
+struct alignas(16) MicroStep {
     uint8_t kind;
     uint8_t nbits;
-    uint16_t op0_code;  // SK_REG: code of ops[op_begin], read with the step (no dependent load)
-    uint32_t op_begin;
-    uint32_t op_count;
+    uint16_t op0_code;  // SK_REG: code of ops[op_begin]; streamed: 64-byte lines of coefficients
+    uint32_t op_begin;  // streamed: first word in Plan::raw of the op codes (StreamCode), four to a
+                        // word, SC_END after the last
+    uint32_t op_count;  // streamed: its SC_PHASE ops are the pass's phases from this one on
     uint32_t coef;     // SK_GENERIC: matrix offset (complex elements); SK_MFMA*: operand offset in
-                       // Plan::raw; SK_REG: coefficient offset of ops[op_begin]
+                       // Plan::raw; SK_REG: coefficient offset of ops[op_begin]; streamed: of the first op
+    // SK_REG: pcols and tcols as LDS byte offsets after the tile's XOR
+    // swizzle (the swizzle is linear over GF(2), so the byte offset of a
+    // register amplitude is the XOR of these).  Streamed steps write register
+    // s at the XOR of wbyte over its bits and wflip instead of pbyte.
+    uint32_t pbyte[4];
+    uint32_t wbyte[4];
+    uint32_t wflip;
+    uint32_t tbyte[12];
+    uint32_t phase_coef;  // streamed: thread tables of its SC_PHASE ops
+    uint32_t pad_[2];
     uint8_t bits[16];  // SK_REG: ascending tile bits; SK_GENERIC/SK_MFMA: tile bit of matrix bit i
     // Layout of the LDS tile when the step runs: the amplitude of tile index
     // y sits at LDS index XOR_{b in y} cols[b] (linear over GF(2); CNOTs are
@@ -59,11 +98,6 @@ struct MicroStep {
     // SK_MFMA: layout columns of matrix bit i (gcols) and, in tcols, of the
     // non-gate tile bits in ascending order (the columns of the contraction).
     uint16_t gcols[8];
-    // SK_REG: tcols and pcols as LDS byte offsets after the tile's XOR
-    // swizzle (the swizzle is linear over GF(2), so the byte offset of a
-    // register amplitude is the XOR of these).
-    uint32_t tbyte[12];
-    uint32_t pbyte[4];
 };
 
 constexpr int kMaxQubits = 40;
@@ -104,6 +138,9 @@ struct PassArgs {
     // amplitudes written to 2^low-amplitude runs of the other, through
     // Plan::scatter_args[scatter_idx].
     uint8_t scatter;
+    // The pass runs on k_stream: its steps are streams of rotations and
+    // diagonals.
+    uint8_t stream;
     uint64_t first_g[16];
     uint64_t last_g[16];
     uint64_t synth_index;
@@ -112,6 +149,9 @@ struct PassArgs {
     uint64_t zero_mask;
     uint32_t scatter_idx;
     uint32_t scatter_pad;
+    uint32_t phase_begin;  // streamed: its phases in Plan::phases
+    uint32_t phase_count;
+    uint64_t last_xor;  // streamed direct last step: XORed into every stored offset
 };
 
 // Store side of a scatter pass: store index bit k of a tile goes to state
@@ -167,6 +207,8 @@ struct PlanOptions {
     bool reorder = true;     // swap-free programs: also plan the gates in a canonical order, keep the cheaper
     bool scatter = false;    // 2+ trailing permutation passes become one out-of-place pass (needs a second buffer)
     bool relabel = false;    // with scatter: passes after the support region read contiguous tiles (relabelled qubits)
+    bool stream = false;     // streamed passes (k_stream) where every gate allows; 4-bit micro-steps only
+    bool phases = true;      // with stream: CRk gates need only one of their qubits in registers
     bool zero_start = true;  // the first pass sees |0...0> (false: any state, e.g. a product input; no support region)
 };
 
@@ -178,7 +220,8 @@ struct Plan {
     std::vector<MicroStep> micro;
     std::vector<MicroOp> ops;
     std::vector<double> coef;  // interleaved complex128; converted per dtype on upload
-    std::vector<uint32_t> raw; // matrix-core operands, uploaded bit for bit
+    std::vector<uint32_t> raw; // matrix-core operands and streamed op codes, uploaded bit for bit
+    std::vector<Phase> phases; // tile factors of the SC_PHASE ops, pass by pass
     int gate_passes = 0;
     int remap_passes = 0;
     int low_qubits = 0;  // qubits 0..low-1 in every gate tile (as planned)

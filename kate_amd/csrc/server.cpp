@@ -101,7 +101,7 @@ struct Request {
     // arena ranges
     uint64_t off = 0, bytes = 0;
     uint64_t o_state = 0, o_micro = 0, o_ops = 0, o_coef = 0, o_raw = 0, o_scratch = 0,
-             o_factors = 0, o_state2 = 0, o_scatter = 0;
+             o_factors = 0, o_state2 = 0, o_scatter = 0, o_phases = 0;
     std::vector<float> coef32;
     int stream = -1;
     hipEvent_t done_ev = nullptr;
@@ -181,6 +181,7 @@ uint64_t layout(kate_server* s, Request& r)
     r.o_raw = take(r.plan.raw.size() * sizeof(uint32_t));
     r.o_scratch = take(kate::reduce_scratch_doubles(r.plan.nq_int) * sizeof(double));
     r.o_factors = take(4 * (uint64_t)r.plan.nq_int * sizeof(double));
+    r.o_phases = take(r.plan.phases.size() * sizeof(kate::Phase));
     if (!r.plan.scatter_args.empty()) {  // out-of-place passes: a second state buffer
         r.o_state2 = take((1ull << r.plan.nq_int) * s->amp);
         r.o_scatter = take(r.plan.scatter_args.size() * sizeof(kate::ScatterArgs));
@@ -212,6 +213,9 @@ int launch_request(kate_server* s, Request& r)
     if (!r.plan.raw.empty())
         SV(hipMemcpyAsync(base + r.o_raw, r.plan.raw.data(), r.plan.raw.size() * sizeof(uint32_t),
                           hipMemcpyHostToDevice, st));
+    if (!r.plan.phases.empty())
+        SV(hipMemcpyAsync(base + r.o_phases, r.plan.phases.data(), r.plan.phases.size() * sizeof(kate::Phase),
+                          hipMemcpyHostToDevice, st));
     if (!r.plan.scatter_args.empty())
         SV(hipMemcpyAsync(base + r.o_scatter, r.plan.scatter_args.data(),
                           r.plan.scatter_args.size() * sizeof(kate::ScatterArgs), hipMemcpyHostToDevice, st));
@@ -228,7 +232,8 @@ int launch_request(kate_server* s, Request& r)
     // support (no init kernel); a product state is read as written
     const bool from_zero = r.product.empty();
     kate::DevPlan dp{(const kate::MicroStep*)(base + r.o_micro), (const kate::MicroOp*)(base + r.o_ops),
-                     base + r.o_coef, (const uint32_t*)(base + r.o_raw)};
+                     base + r.o_coef, (const uint32_t*)(base + r.o_raw), nullptr, nullptr,
+                     (const kate::Phase*)(base + r.o_phases)};
     // an out-of-place pass (relabelled, or storing through the trailing
     // permutation) writes the other buffer, which then holds the state
     void* other = r.plan.scatter_args.empty() ? nullptr : base + r.o_state2;
@@ -413,6 +418,7 @@ int kate_server_create(const kate_server_options* options, kate_server** out)
     std::string err = kate::plan_options(ko, po);
     if (!err.empty()) return sfail(KATE_ERR_ARG, err);
     po.scatter = false;  // set per request, by size
+    po.stream = kate::may_stream(ko, po);
     if (po.auto_tile) {
         // one tile size, planned once per request on the scheduler thread:
         // 12-qubit tiles (a mix of 128 circuits of 12..30 qubits at

@@ -164,6 +164,7 @@ struct kate_sim {
     kate::MicroOp* d_ops = nullptr;
     void* d_coef = nullptr;
     uint32_t* d_raw = nullptr;
+    kate::Phase* d_phases = nullptr;
     double* d_scratch = nullptr;
     double* d_out = nullptr;
     double* h_out = nullptr;  // pinned: the reductions write their results here
@@ -205,6 +206,7 @@ void release(kate_sim* s)
     (void)hipFree(s->d_ops);
     (void)hipFree(s->d_coef);
     (void)hipFree(s->d_raw);
+    (void)hipFree(s->d_phases);
     (void)hipFree(s->d_scratch);
     (void)hipFree(s->d_out);
     (void)hipHostFree(s->h_out);
@@ -244,7 +246,7 @@ int launch_plan_pass(kate_sim* s, const kate::PassArgs& pa, const kate::DevPlan&
 int run_passes(kate_sim* s, bool from_zero = false, size_t begin = 0, size_t end = (size_t)-1,
                hipEvent_t* after = nullptr, uint64_t* tiles = nullptr)
 {
-    kate::DevPlan dp{s->d_micro, s->d_ops, s->d_coef, s->d_raw};
+    kate::DevPlan dp{s->d_micro, s->d_ops, s->d_coef, s->d_raw, nullptr, nullptr, s->d_phases};
     end = std::min(end, s->plan.passes.size());
     for (size_t i = begin; i < end; i++) {
         const kate::PassArgs pa = from_zero ? kate::zero_start_pass(s->plan, i, s->support, end) : s->plan.passes[i];
@@ -403,6 +405,12 @@ std::string plan_options(const kate_options& opt, kate::PlanOptions& po)
     if (opt.batch_wgs_per_cu < 0 || opt.batch_wgs_per_cu > 32) return "batch_wgs_per_cu must be in 0..32";
     return "";
 }
+
+bool may_stream(const kate_options& opt, const kate::PlanOptions& po)
+{
+    return opt.tile_qubits == 0 && opt.low_qubits == 0 && opt.use_mfma == 0 && po.micro_bits == 4 && po.euler &&
+           po.factor && po.direct;
+}
 }  // namespace kate
 using kate::plan_options;
 
@@ -516,6 +524,9 @@ int kate_sim_create(const kate_program* program, const kate_options* options, ka
     }
     s->support = po.support;
     s->defer = po.defer;
+    // shapes left to the planner: streamed passes where the gates allow (the
+    // device-free plan text describes the passes without them)
+    po.stream = kate::may_stream(opt, po);
     if (po.scatter) {
         // the scatter pass needs a second state buffer: only when the GPU
         // has room for both and 1 GiB to spare
@@ -561,6 +572,7 @@ int kate_sim_create(const kate_program* program, const kate_options* options, ka
     if (rc == KATE_OK) rc = upload(&s->d_micro, s->plan.micro, s->stream);
     if (rc == KATE_OK) rc = upload(&s->d_ops, s->plan.ops, s->stream);
     if (rc == KATE_OK) rc = upload(&s->d_raw, s->plan.raw, s->stream);
+    if (rc == KATE_OK && !s->plan.phases.empty()) rc = upload(&s->d_phases, s->plan.phases, s->stream);
     if (rc == KATE_OK) {
         if (s->dtype == KATE_C128) {
             rc = upload((double**)&s->d_coef, s->plan.coef, s->stream);
@@ -630,7 +642,7 @@ int kate_sim_run_timed(kate_sim* s, float* pass_ms, int32_t* pass_is_remap, int3
     int rc = KATE_OK;
     for (auto& e : ev)
         if (rc == KATE_OK && hipEventCreate(&e) != hipSuccess) rc = fail(KATE_ERR_HIP, "hipEventCreate");
-    kate::DevPlan dp{s->d_micro, s->d_ops, s->d_coef, s->d_raw};
+    kate::DevPlan dp{s->d_micro, s->d_ops, s->d_coef, s->d_raw, nullptr, nullptr, s->d_phases};
     if (rc == KATE_OK && hipEventRecord(ev[0], s->stream) != hipSuccess) rc = fail(KATE_ERR_HIP, "hipEventRecord");
     for (size_t i = 0; i < np && rc == KATE_OK; i++) {
         int e = launch_plan_pass(s, s->plan.passes[i], dp);
@@ -907,7 +919,8 @@ int kate_sim_stream(kate_sim* s, void** stream)
 int kate_sim_describe(kate_sim* s, char* buf, size_t len)
 {
     if (!s || !buf || !len) return fail(KATE_ERR_ARG, "null argument");
-    std::string d = s->plan.describe();
+    const char* v = std::getenv("KATE_DESCRIBE_OPS");  // as kate_plan_describe
+    std::string d = s->plan.describe(v && v[0] == '1');
     std::strncpy(buf, d.c_str(), len - 1);
     buf[len - 1] = 0;
     return d.size() < len ? KATE_OK : fail(KATE_ERR_ARG, "buffer too small");
