@@ -148,9 +148,9 @@ enum {
        plans of 12-qubit tiles or narrower; needs the second buffer as
        KATE_PLAN_NO_SCATTER describes; results bit for bit the same) */
     KATE_PLAN_NO_RELABEL = 256,
-    /* keep dense 5-qubit gates of a KATE_C64 plan on the VALU (register
-       blocks) instead of the FP32 matrix cores, which take them by default
-       (use_mfma = 0); results to FP32 rounding */
+    /* keep dense gates off the matrix cores (use_mfma = 0), which by default
+       take those of 4 to 6 qubits in the state's own precision (a batch
+       keeps them on the VALU); results to rounding */
     KATE_PLAN_NO_MATRIX5 = 512
 };
 

@@ -335,8 +335,7 @@ class Simulator:
         `scatter=False` runs the trailing permutation passes as planned
         instead of as one out-of-place pass; `relabel=False` keeps every
         pass in place on the virtual qubit order; `matrix5=False` keeps dense
-        5-qubit gates of a complex64 state on the VALU instead of the matrix
-        cores."""
+        gates of 4 to 6 qubits on the VALU instead of the matrix cores."""
         self.n = circuit.n
         self.dtype = {"c128": KATE_C128, "c64": KATE_C64}[dtype]
         self.amp = np.complex128 if self.dtype == KATE_C128 else np.complex64

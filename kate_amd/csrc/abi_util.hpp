@@ -13,4 +13,7 @@ std::string plan_options(const kate_options& opt, PlanOptions& po);
 // Whether every shape and form is left to the planner, so that it may use
 // streamed passes (PlanOptions::stream).
 bool may_stream(const kate_options& opt, const PlanOptions& po);
+// Whether dense gates of 5 and 6 qubits may run on the matrix cores
+// (PlanOptions::gate_mfma).
+bool may_gate_mfma(const kate_options& opt, const PlanOptions& po);
 }  // namespace kate

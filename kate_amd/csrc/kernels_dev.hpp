@@ -457,76 +457,120 @@ __device__ __forceinline__ void dense5(Cx<R>* tile, const MicroStep* __restrict_
     }
 }
 
-// WIDE instantiations also run SK_GENERIC micro-steps; keeping them out of
-// the common variant keeps its register count at two waves per SIMD.
+// WIDE: kRegSteps instantiations run register steps only, kGateSteps ones also
+// SK_MFMA steps, kAnySteps ones every kind; keeping the larger steps out of the
+// common variants keeps their register counts at the waves per SIMD that LDS
+// allows.
+enum StepSet { kRegSteps = 0, kAnySteps = 1, kGateSteps = 2 };
+
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// Dense K-qubit gate (K = 4 or 5) on the matrix cores, complex64 tile.
-// The gate is a real 2D x 2D matrix (D = 2^K) in the embedding
-// [Yr; Yi] = [[Mr, -Mi], [Mi, Mr]] [Xr; Xi], with the contraction index
-// ordered (gate row g, re/im) so each lane reads one float of X per step.
-// The tile is the 2D x 2^(TB-K) right-hand side; each wave owns whole
-// 32-column blocks, so it reads and overwrites only its own columns.
-// A is pre-arranged on the host in lane order: A[(rb*D + s)*64 + lane] =
-// A'[rb*32 + lane%32][2s + lane/32] for v_mfma_f32_32x32x2f32.
-template <int TB, int K>
-__device__ __forceinline__ void mfma_dense(Cx<float>* tile, const MicroStep* __restrict__ msp,
-                                           const float* __restrict__ A)
+template <typename R>
+__device__ __forceinline__ Cx<R>& lds_at(Cx<R>* tile, uint32_t byte_off);
+
+template <typename R>
+struct MfmaVec;
+template <>
+struct MfmaVec<double> {
+    typedef double t __attribute__((ext_vector_type(4)));
+};
+template <>
+struct MfmaVec<float> {
+    typedef float t __attribute__((ext_vector_type(4)));
+};
+
+// 16x16 += 16x4 * 4x16, one entry of each operand per lane.
+__device__ __forceinline__ MfmaVec<double>::t mfma_16x16x4(double a, double b, MfmaVec<double>::t c)
 {
-    constexpr int D = 1 << K;
-    constexpr int RB = 2 * D / 32;
-    constexpr int NW = (1 << (TB - 4)) / 64;
-    constexpr int CB = (1 << (TB - K)) / 32;
-    constexpr int CBW = CB / NW;
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ MfmaVec<float>::t mfma_16x16x4(float a, float b, MfmaVec<float>::t c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Dense K-qubit gate on the matrix cores, in the state's own precision.  The
+// gate is a real 2D x 2D matrix (D = 2^K) in the embedding
+// [[Mr, -Mi], [Mi, Mr]] and the tile the 2D x 2^(TB-K) right-hand side.  A
+// wave owns blocks of 16 columns, which it reads and overwrites in place
+// (no barrier inside the step), and takes all rows of them: each element of
+// A is then loaded once per wave and used for all its column blocks.
+// Contraction step 2t + p holds part p (re, im) of gate rows 4t + lane/16, so
+// a lane's two operands of B are one amplitude, and the rows of A are ordered
+// so that an amplitude's two parts come out in one lane: whole amplitudes are
+// read from and written to LDS.  Row i of row block b is in lane group i % 4,
+// element i / 4 (double), or lane group i / 4, element i % 4 (float).
+// A is in lane order (add_gate_operand): two values per lane, the parts
+// p = 0, 1, for each t and row block.
+// Bound by the matrix cores in complex128 (K = 5: 8192 clocks of a CU's FP64
+// peak per 12-qubit tile, its HBM traffic 6000) and about evenly by HBM in
+// complex64.  26 qubits, 24 Haar gates, all passes: K = 5 complex128 13.1 ms
+// (register blocks on the VALU, matrix rows by scalar loads) -> 5.5, complex64
+// 3.80 (32x32x2 products, single components scattered to LDS, two waves per
+// SIMD) -> 3.26; K = 4 (register ops) 2.34 -> 2.07 and 1.37 -> 1.10; 23 qubits,
+// K = 6 (generic step) 36.7 -> 2.9 and 36.7 -> 1.0.
+template <typename R, int TB, int NB, int K>
+__device__ __forceinline__ void mfma_gate(Cx<R>* tile, const MicroStep* __restrict__ msp, const R* __restrict__ A)
+{
+    typedef typename MfmaVec<R>::t V4;
+    constexpr int D = 1 << K, RB = 2 * D / 16, T = D / 4;
+    constexpr int NW = (1 << (TB - NB)) / 64, CB = (1 << (TB - K)) / 16, CBW = CB / NW;
     static_assert(CBW >= 1 && CBW * NW == CB, "column blocks must split evenly over the waves");
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t half = (uint32_t)lane >> 5;
-    float* tf = reinterpret_cast<float*>(tile);
-    float a[RB][D];
-#pragma unroll
-    for (int rb = 0; rb < RB; rb++)
-#pragma unroll
-        for (int s = 0; s < D; s++) a[rb][s] = A[(rb * D + s) * 64 + lane];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, q = lane >> 4;
     uint32_t gc[K];
 #pragma unroll
-    for (int i = 0; i < K; i++) gc[i] = msp->gcols[i];
+    for (int i = 0; i < K; i++) gc[i] = swz<R>(msp->gcols[i]) * (uint32_t)sizeof(Cx<R>);
+    // LDS byte offset of the lane's column in each block
+    uint32_t col[CBW];
 #pragma unroll
-    for (int cbi = 0; cbi < CBW; cbi++) {
-        const uint32_t col = (uint32_t)(wave * CBW + cbi) * 32u + (uint32_t)(lane & 31);
-        uint32_t lq = 0;
+    for (int c = 0; c < CBW; c++) {
+        const uint32_t j = (wave * CBW + c) * 16u + (lane & 15u);
+        uint32_t l = 0;
 #pragma unroll
-        for (int j = 0; j < TB - K; j++)
-            if ((col >> j) & 1u) lq ^= msp->tcols[j];
-        f32x16 acc[RB];
-#pragma unroll
-        for (int rb = 0; rb < RB; rb++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[rb][r] = 0.0f;
-#pragma unroll
-        for (int s = 0; s < D; s++) {
-            uint32_t lp = lq;
-#pragma unroll
-            for (int i = 0; i < K; i++)
-                if ((s >> i) & 1) lp ^= gc[i];
-            const float b = tf[2 * swz<float>(lp) + half];
-#pragma unroll
-            for (int rb = 0; rb < RB; rb++) acc[rb] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[rb][s], b, acc[rb], 0, 0, 0);
-        }
-        // acc[rb][r] holds output row rb*32 + 8(r/4) + 4*half + r%4 of this lane's column
-#pragma unroll
-        for (int rb = 0; rb < RB; rb++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int o0 = rb * 32 + 8 * (r / 4) + (r % 4);  // row without the lane-half bit (bit 2)
-                const int g0 = o0 % D;
-                uint32_t lp = lq;
-#pragma unroll
-                for (int i = 0; i < K; i++)
-                    if (i != 2 && ((g0 >> i) & 1)) lp ^= gc[i];
-                if (half) lp ^= gc[2];
-                tf[2 * swz<float>(lp) + (uint32_t)(o0 / D)] = acc[rb][r];
-            }
+        for (int i = 0; i < TB - K; i++)
+            if ((j >> i) & 1u) l ^= msp->tcols[i];
+        col[c] = swz<R>(l) * (uint32_t)sizeof(Cx<R>);
     }
+    V4 acc[CBW][RB];
+#pragma unroll
+    for (int c = 0; c < CBW; c++)
+#pragma unroll
+        for (int b = 0; b < RB; b++) acc[c][b] = V4{0, 0, 0, 0};
+    const uint32_t rd = ((q & 1u) ? gc[0] : 0u) ^ ((q & 2u) ? gc[1] : 0u);
+    const Cx<R>* __restrict__ a2 = reinterpret_cast<const Cx<R>*>(A) + lane;
+#pragma unroll 2
+    for (int t = 0; t < T; t++) {
+        uint32_t row = rd;
+#pragma unroll
+        for (int i = 2; i < K; i++)
+            if ((t >> (i - 2)) & 1) row ^= gc[i];
+        Cx<R> x[CBW];
+#pragma unroll
+        for (int c = 0; c < CBW; c++) x[c] = lds_at(tile, col[c] ^ row);
+#pragma unroll
+        for (int b = 0; b < RB; b++) {
+            const Cx<R> a = a2[(t * RB + b) * 64];
+#pragma unroll
+            for (int c = 0; c < CBW; c++) acc[c][b] = mfma_16x16x4(a.re, x[c].re, acc[c][b]);
+#pragma unroll
+            for (int c = 0; c < CBW; c++) acc[c][b] = mfma_16x16x4(a.im, x[c].im, acc[c][b]);
+        }
+    }
+    // rows of block b: double 8b + 4h + q, float 8b + 2q + h
+    constexpr bool F64 = sizeof(R) == 8;
+    const uint32_t wr = F64 ? rd : ((q & 1u) ? gc[1] : 0u) ^ ((q & 2u) ? gc[2] : 0u);
+#pragma unroll
+    for (int c = 0; c < CBW; c++)
+#pragma unroll
+        for (int b = 0; b < RB; b++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                uint32_t row = wr ^ (h ? (F64 ? gc[2] : gc[0]) : 0u);
+#pragma unroll
+                for (int i = 3; i < K; i++)
+                    if ((b >> (i - 3)) & 1) row ^= gc[i];
+                lds_at(tile, col[c] ^ row) = Cx<R>{acc[c][b][2 * h], acc[c][b][2 * h + 1]};
+            }
 }
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -535,7 +579,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-// mfma_dense with split-bf16 products: A = Ahi + Alo (split on the host),
+// A 4- or 5-qubit gate (complex64) with split-bf16 products: A = Ahi + Alo (split on the host),
 // B = Bhi + Blo (split here), acc += Ahi Bhi + Ahi Blo + Alo Bhi on
 // v_mfma_f32_32x32x16_bf16 (lane l holds contraction indices 8(l/32)..+7 of
 // its row / column).  Eight consecutive contraction indices are four complex
@@ -764,7 +808,7 @@ __device__ __forceinline__ uint64_t direct_reg_offset(const uint64_t* __restrict
     return off;
 }
 
-template <typename R, int TB, bool WIDE, int NB, bool LIGHT>
+template <typename R, int TB, int WIDE, int NB, bool LIGHT>
 __device__ __forceinline__ void run_steps(const PassArgs& pa, Cx<R>* tile, const MicroStep* __restrict__ micro,
                                           const MicroOp* __restrict__ ops, const Cx<R>* __restrict__ coef,
                                           const uint32_t* __restrict__ raw, uint32_t m_begin, uint32_t m_end)
@@ -783,27 +827,30 @@ __device__ __forceinline__ void run_steps(const PassArgs& pa, Cx<R>* tile, const
             const uint32_t bw = b ^ reg_offset<NB>((int)f, oc);
 #pragma unroll
             for (int s = 0; s < N; s++) lds_at(tile, bw ^ reg_offset<NB>(s, oc)) = v[s];
-        } else if (WIDE) {
-            // (a 1024-thread workgroup is held to 128 VGPRs: too few for
-            // dense5's 32 amplitudes in complex128)
-            constexpr bool kDense5 = sizeof(R) == 4 || (TB - NB) <= 9;
-            if (kDense5 && msp->kind == SK_GENERIC && msp->nbits == 5) {
-                dense5<R, TB, NB>(tile, msp, coef + msp->coef);
-            } else if constexpr (sizeof(R) == 4 && NB == 4) {
-                Cx<float>* tf = reinterpret_cast<Cx<float>*>(tile);
-                if (msp->kind == SK_MFMA) {
-                    const float* A = reinterpret_cast<const float*>(raw + msp->coef);
-                    if (msp->nbits == 5) mfma_dense<TB, 5>(tf, msp, A);
-                    else mfma_dense<TB, 4>(tf, msp, A);
-                } else if (msp->kind == SK_MFMA_BF16) {
-                    if (msp->nbits == 5) mfma_bf16<TB, 5>(tf, msp, raw + msp->coef);
-                    else mfma_bf16<TB, 4>(tf, msp, raw + msp->coef);
+        } else if constexpr (WIDE != kRegSteps && NB == 4) {
+            const R* operand = reinterpret_cast<const R*>(raw + msp->coef);
+            const bool gate = WIDE == kGateSteps || msp->kind == SK_MFMA;
+            if (gate && msp->nbits == 5) mfma_gate<R, TB, NB, 5>(tile, msp, operand);
+            else if (gate && msp->nbits == 6) mfma_gate<R, TB, NB, 6>(tile, msp, operand);
+            else if (gate) mfma_gate<R, TB, NB, 4>(tile, msp, operand);
+            else if constexpr (WIDE == kAnySteps) {
+                if (msp->kind == SK_MFMA_BF16) {
+                    if constexpr (sizeof(R) == 4) {
+                        if (msp->nbits == 5) mfma_bf16<TB, 5>(tile, msp, raw + msp->coef);
+                        else mfma_bf16<TB, 4>(tile, msp, raw + msp->coef);
+                    }
+                } else if (msp->nbits == 5) {
+                    dense5<R, TB, NB>(tile, msp, coef + msp->coef);
                 } else {
                     generic_dense<R, TB, NB>(tile, msp, coef + msp->coef);
                 }
-            } else {
-                generic_dense<R, TB, NB>(tile, msp, coef + msp->coef);
             }
+        } else if constexpr (WIDE != kRegSteps) {
+            // (a 1024-thread workgroup is held to 128 VGPRs: too few for
+            // dense5's 32 amplitudes in complex128)
+            constexpr bool kDense5 = TB - NB <= 9;
+            if (kDense5 && msp->nbits == 5) dense5<R, TB, NB>(tile, msp, coef + msp->coef);
+            else generic_dense<R, TB, NB>(tile, msp, coef + msp->coef);
         }
         __syncthreads();
     }
@@ -894,7 +941,7 @@ __device__ __forceinline__ void scatter_store(Cx<R>* __restrict__ dst, const Pas
     }
 }
 
-template <typename R, int TB, bool WIDE, int NB, bool LIGHT>
+template <typename R, int TB, int WIDE, int NB, bool LIGHT>
 __device__ __forceinline__ void tile_pass(Cx<R>* __restrict__ state, const PassArgs& pa, uint64_t blk, Cx<R>* tile,
                                           const MicroStep* __restrict__ micro, const MicroOp* __restrict__ ops,
                                           const Cx<R>* __restrict__ coef, const uint32_t* __restrict__ raw,
@@ -1017,18 +1064,18 @@ constexpr int kLdsWavesPerSimd =
 
 // Minimum waves per SIMD the register allocation must allow: two for
 // complex128 16-amplitude threads (their 64 KiB LDS tiles allow two per CU),
-// for the other light variants as many as their LDS tiles allow, at most
-// four; the compiler's own choice otherwise.
-template <typename R, int TB, int NB, bool LIGHT>
+// for the other light variants and the complex64 gate variant (176 VGPRs left
+// it two waves) as many as their LDS tiles allow, at most four; the compiler's own choice otherwise.
+template <typename R, int TB, int WIDE, int NB, bool LIGHT>
 constexpr int kPassWavesPerEU =
     (sizeof(R) == 8 && NB == 4) ? 2
-                                : (LIGHT ? (kLdsWavesPerSimd<R, TB, NB> < 1 ? 1
+                                : (LIGHT || WIDE == kGateSteps ? (kLdsWavesPerSimd<R, TB, NB> < 1 ? 1
                                             : (kLdsWavesPerSimd<R, TB, NB> > 4 ? 4 : kLdsWavesPerSimd<R, TB, NB>))
                                          : 1);
 
 // LIGHT: the pass's ops are all in the light set (apply_op_light).
-template <typename R, int TB, bool WIDE, int NB, bool LIGHT>
-__global__ __launch_bounds__(1 << (TB - NB)) __attribute__((amdgpu_waves_per_eu(kPassWavesPerEU<R, TB, NB, LIGHT>)))
+template <typename R, int TB, int WIDE, int NB, bool LIGHT>
+__global__ __launch_bounds__(1 << (TB - NB)) __attribute__((amdgpu_waves_per_eu(kPassWavesPerEU<R, TB, WIDE, NB, LIGHT>)))
 void k_pass(Cx<R>* __restrict__ state, PassArgs pa,
                                                          const MicroStep* __restrict__ micro,
                                                          const MicroOp* __restrict__ ops,
@@ -1358,10 +1405,10 @@ int stream_r(int tile_bits, void* state, const PassArgs& pa, const DevPlan& dp, 
 // runs out sets *err instead of spinning on.
 // complex64 register-step batch kernels are held to 128 VGPRs (4 waves per
 // SIMD): with 137 the 8-wave workgroups of 13-bit tiles ran one per CU.
-template <typename R, bool WIDE>
+template <typename R, int WIDE>
 constexpr int kBatchWavesPerEU = (sizeof(R) == 4 && !WIDE) ? 4 : 1;
 
-template <typename R, int TB, bool WIDE, int NB>
+template <typename R, int TB, int WIDE, int NB>
 __global__ __launch_bounds__(1 << (TB - NB)) __attribute__((amdgpu_waves_per_eu(kBatchWavesPerEU<R, WIDE>)))
 void k_batch(Cx<R>* __restrict__ states,
                                                          const uint64_t* __restrict__ circ_off,
@@ -1441,14 +1488,21 @@ int pass_t(void* state, int nq_int, const PassArgs& pa, const DevPlan& dp, hipSt
     // one workgroup per tile; a run from |0...0> may list fewer rest qubits
     (void)nq_int;
     const unsigned grid = 1u << pa.nrest;
-    if (pa.has_wide)
-        hipLaunchKernelGGL((k_pass<R, TB, true, NB, false>), dim3(grid), dim3(1 << (TB - NB)), 0, s, (Cx<R>*)state,
+    if (pa.has_wide == kGateSteps) {
+        if constexpr (NB == 4)
+            hipLaunchKernelGGL((k_pass<R, TB, kGateSteps, NB, false>), dim3(grid), dim3(1 << (TB - NB)), 0, s,
+                               (Cx<R>*)state, pa, dp.micro, dp.ops, (const Cx<R>*)dp.coef, dp.raw, (Cx<R>*)dp.dst,
+                               dp.scatter);
+        else
+            return (int)hipErrorInvalidValue;
+    } else if (pa.has_wide)
+        hipLaunchKernelGGL((k_pass<R, TB, kAnySteps, NB, false>), dim3(grid), dim3(1 << (TB - NB)), 0, s, (Cx<R>*)state,
                            pa, dp.micro, dp.ops, (const Cx<R>*)dp.coef, dp.raw, (Cx<R>*)dp.dst, dp.scatter);
     else if (pa.light)
-        hipLaunchKernelGGL((k_pass<R, TB, false, NB, true>), dim3(grid), dim3(1 << (TB - NB)), 0, s, (Cx<R>*)state,
+        hipLaunchKernelGGL((k_pass<R, TB, kRegSteps, NB, true>), dim3(grid), dim3(1 << (TB - NB)), 0, s, (Cx<R>*)state,
                            pa, dp.micro, dp.ops, (const Cx<R>*)dp.coef, dp.raw, (Cx<R>*)dp.dst, dp.scatter);
     else
-        hipLaunchKernelGGL((k_pass<R, TB, false, NB, false>), dim3(grid), dim3(1 << (TB - NB)), 0, s, (Cx<R>*)state,
+        hipLaunchKernelGGL((k_pass<R, TB, kRegSteps, NB, false>), dim3(grid), dim3(1 << (TB - NB)), 0, s, (Cx<R>*)state,
                            pa, dp.micro, dp.ops, (const Cx<R>*)dp.coef, dp.raw, (Cx<R>*)dp.dst, dp.scatter);
     return (int)hipGetLastError();
 }
@@ -1475,7 +1529,7 @@ int pass_r(int tile_bits, void* state, int nq_int, const PassArgs& pa, const Dev
     }
 }
 
-template <typename R, int TB, bool WIDE, int NB>
+template <typename R, int TB, int WIDE, int NB>
 int batch_t(const BatchArgs& a, hipStream_t s)
 {
     hipLaunchKernelGGL((k_batch<R, TB, WIDE, NB>), dim3(a.grid), dim3(1 << (TB - NB)), 0, s, (Cx<R>*)a.states,
@@ -1484,7 +1538,7 @@ int batch_t(const BatchArgs& a, hipStream_t s)
     return (int)hipGetLastError();
 }
 
-template <typename R, int TB, bool WIDE>
+template <typename R, int TB, int WIDE>
 int batch_nb(const BatchArgs& a, hipStream_t s)
 {
     if constexpr (sizeof(R) == 8)
@@ -1493,7 +1547,7 @@ int batch_nb(const BatchArgs& a, hipStream_t s)
     return batch_t<R, TB, WIDE, 4>(a, s);
 }
 
-template <typename R, bool WIDE>
+template <typename R, int WIDE>
 int batch_w(const BatchArgs& a, hipStream_t s)
 {
     switch (a.tile_bits) {

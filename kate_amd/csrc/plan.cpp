@@ -552,33 +552,37 @@ struct Builder {
     }
 
     // A dense 2^k x 2^k complex matrix (row-major, interleaved) as the lane-
-    // ordered A operand of the SK_MFMA step (kernels.hip mfma_dense):
-    // A[(rb*D + s)*64 + lane] = A'[rb*32 + lane%32][2s + lane/32] with
-    // A'[i][2g] = Mr[i][g], A'[i][2g+1] = -Mi[i][g] for i < D (real rows) and
-    // A'[D+i][2g] = Mi[i][g], A'[D+i][2g+1] = Mr[i][g] (imaginary rows).
-    uint32_t add_mfma_operand(const double* m, int k)
+    // ordered A operand of an SK_MFMA step (kernels_dev.hpp mfma_gate), in the
+    // state's precision: for contraction steps 2t + p, row block b and lane l,
+    // the entry of the real embedding at gate row g = 4t + l/16, part p, and
+    // the output row of index i = l%16: gate row 8b + 4(i/8) + i%4, part
+    // (i/4)%2 (double) or gate row 8b + i/2, part i%2 (float).
+    uint32_t add_gate_operand(const double* m, int k)
     {
-        const int D = 1 << k, RB = 2 * D / 32;
-        std::vector<double> a((size_t)RB * D * 64);
-        for (int rb = 0; rb < RB; rb++)
-            for (int st = 0; st < D; st++)
-                for (int lane = 0; lane < 64; lane++) {
-                    const int i = rb * 32 + lane % 32, kk = 2 * st + lane / 32;
-                    const int g = kk / 2, p = kk % 2;
-                    const int row = i % D;
-                    const double mr = m[2 * ((size_t)row * D + g)], mi = m[2 * ((size_t)row * D + g) + 1];
-                    double v;
-                    if (i < D) v = p == 0 ? mr : -mi;
-                    else v = p == 0 ? mi : mr;
-                    a[(size_t)(rb * D + st) * 64 + lane] = v;
-                }
+        const int D = 1 << k, RB = 2 * D / 16, T = D / 4;
+        const bool f64 = opt.amp_bytes == 16;
+        while (plan.raw.size() % 4) plan.raw.push_back(0);  // 16-byte loads
         const uint32_t off = (uint32_t)plan.raw.size();
-        for (double v : a) {
-            const float f = (float)v;
-            uint32_t u;
-            std::memcpy(&u, &f, 4);
-            plan.raw.push_back(u);
-        }
+        for (int t = 0; t < T; t++)
+            for (int b = 0; b < RB; b++)
+                for (int lane = 0; lane < 64; lane++)
+                    for (int p = 0; p < 2; p++) {
+                        const int i = lane % 16, g = 4 * t + lane / 16;
+                        const int row = f64 ? 8 * b + 4 * (i / 8) + i % 4 : 8 * b + i / 2;
+                        const int part = f64 ? (i / 4) % 2 : i % 2;
+                        const double mr = m[2 * ((size_t)row * D + g)], mi = m[2 * ((size_t)row * D + g) + 1];
+                        const double v = part == p ? mr : (part == 0 ? -mi : mi);
+                        uint32_t w[2];
+                        if (f64) {
+                            std::memcpy(w, &v, 8);
+                            plan.raw.push_back(w[0]);
+                            plan.raw.push_back(w[1]);
+                        } else {
+                            const float f = (float)v;
+                            std::memcpy(w, &f, 4);
+                            plan.raw.push_back(w[0]);
+                        }
+                    }
         return off;
     }
 
@@ -589,7 +593,8 @@ struct Builder {
         return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
     }
 
-    // The same real embedding as add_mfma_operand, split into bf16 hi + lo
+    // The gate's real embedding [[Mr, -Mi], [Mi, Mr]] (contraction index: gate row,
+    // re/im), split into bf16 hi + lo
     // parts and laid out for v_mfma_f32_32x32x16_bf16: for row block rb,
     // K-block t (16 contraction indices) and part (0 hi, 1 lo), lane l holds
     // A'[rb*32 + l%32][16t + 8(l/32) + j], j = 0..7, as four 32-bit words.
@@ -1247,7 +1252,7 @@ struct Builder {
                     if (tile_of[g.q[j]] >= 0) m |= 1ull << tile_of[g.q[j]];
                 tm[i] = m;
                 if (phases) any[i] = g.id == 4;
-                ok[i] = g.k <= nb && !(g.id == 0 && opt.mfma && g.k == 4);
+                ok[i] = g.k <= nb && !(g.id == 0 && (opt.mfma || opt.gate_mfma) && g.k == 4);
                 lazy[i] = g.id == 3;
             }
             if (opt.mfma_fuse) {
@@ -1274,7 +1279,7 @@ struct Builder {
                 std::vector<double> u(2 * (size_t)(1 << w) * (1 << w), 0.0);
                 for (int d = 0; d < (1 << w); d++) u[2 * ((size_t)d * (1 << w) + d)] = 1.0;
                 for (int a : acc) compose_into(u, w, ms.bits, prog.gates[(size_t)rem[(size_t)a]], tile_of);
-                ms.coef = opt.mfma_bf16 ? add_bf16_operand(u.data(), w) : add_mfma_operand(u.data(), w);
+                ms.coef = opt.mfma_bf16 ? add_bf16_operand(u.data(), w) : add_gate_operand(u.data(), w);
                 fill_mfma_cols(ms, cols);
                 plan.micro.push_back(ms);
                 std::vector<int> next;
@@ -1313,12 +1318,16 @@ struct Builder {
                 // the first remaining gate is one the register path does not take
                 const PlanGate& g = prog.gates[(size_t)rem[0]];
                 if (g.id != 0) return "internal: non-dense gate left out of micro-steps";
-                const bool matrix = (opt.mfma && g.k >= 4 && g.k <= 5) || (opt.mfma5 && g.k == 5);
-                ms.kind = matrix ? (opt.mfma_bf16 ? SK_MFMA_BF16 : SK_MFMA) : SK_GENERIC;
+                // gates of 4 to 6 qubits (gate_mfma): one of 3 fits the
+                // register path's HBM time, wider ones leave fewer columns
+                // than a wave's blocks (times at mfma_gate)
+                const bool matrix = (opt.mfma && g.k >= 4 && g.k <= 5) || (opt.mfma5 && g.k == 5) ||
+                                    (opt.gate_mfma && g.k >= 4 && g.k <= 6);
+                ms.kind = matrix ? (opt.mfma_bf16 && g.k <= 5 ? SK_MFMA_BF16 : SK_MFMA) : SK_GENERIC;
                 ms.nbits = (uint8_t)g.k;
                 for (int i = 0; i < g.k; i++) ms.bits[i] = (uint8_t)tile_of[g.q[i]];
                 if (ms.kind == SK_MFMA || ms.kind == SK_MFMA_BF16) {
-                    ms.coef = ms.kind == SK_MFMA ? add_mfma_operand(prog.mat.data() + 2 * g.moff, g.k)
+                    ms.coef = ms.kind == SK_MFMA ? add_gate_operand(prog.mat.data() + 2 * g.moff, g.k)
                                                  : add_bf16_operand(prog.mat.data() + 2 * g.moff, g.k);
                     fill_mfma_cols(ms, cols);
                 } else {
@@ -1418,7 +1427,8 @@ struct Builder {
         pa.light = 1;
         for (uint32_t m = pa.micro_begin; m < plan.micro.size(); m++) {
             const MicroStep& ms = plan.micro[m];
-            if (ms.kind != SK_REG) pa.has_wide = 1;
+            if (ms.kind == SK_MFMA && !pa.has_wide) pa.has_wide = 2;
+            else if (ms.kind != SK_REG && ms.kind != SK_MFMA) pa.has_wide = 1;
             for (uint32_t o = ms.op_begin; !pa.stream && ms.kind == SK_REG && o < ms.op_begin + ms.op_count; o++)
                 if (!light_op(plan.ops[o].code)) pa.light = 0;
         }
@@ -2084,7 +2094,7 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
     plan.tile_bits = std::min(opt.tile_bits, plan.nq_int);
     if (opt.micro_bits != 3 && opt.micro_bits != 4) return "micro-steps have 3 or 4 bits";
     if (opt.amp_bytes != 16 && opt.amp_bytes != 8) return "amplitudes have 8 or 16 bytes";
-    if (opt.micro_bits != 4 && (opt.mfma || opt.mfma_fuse || opt.mfma5)) return "matrix-core steps need 4-bit micro-steps";
+    if (opt.micro_bits != 4 && (opt.mfma || opt.mfma_fuse || opt.mfma5 || opt.gate_mfma)) return "matrix-core steps need 4-bit micro-steps";
     Builder b{prog, opt, plan};
     if (opt.stream && opt.phases && opt.micro_bits == 4) {
         // a program of gates that can all be streamed, CRk among them

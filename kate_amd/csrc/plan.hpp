@@ -28,7 +28,7 @@ enum OpKind : uint16_t {
 enum StepKind : uint8_t {
     SK_REG = 0,      // 4 tile bits held in registers, ops applied in place
     SK_GENERIC = 1,  // one dense gate of any size, matrix-vector on the LDS tile
-    SK_MFMA = 2,     // one dense gate of 4 or 5 qubits on matrix cores (complex64, FP32 products)
+    SK_MFMA = 2,     // one dense gate of 4 to 6 qubits on matrix cores, in the state's precision
     SK_MFMA_BF16 = 3,  // the same with split-bf16 products (x = hi + lo, three products), FP32 accumulation
 };
 
@@ -112,7 +112,7 @@ struct PassArgs {
     uint8_t load_pos[16];
     uint8_t store_pos[16];
     uint8_t rest_pos[kMaxQubits];
-    uint8_t has_wide;    // some micro-step is not SK_REG (selects the kernel variant)
+    uint8_t has_wide;    // selects the kernel variant: 0 every micro-step is SK_REG, 2 also SK_MFMA ones, 1 any
     uint8_t micro_bits;  // bits per register micro-step (3 or 4): 2^micro_bits amplitudes per thread
     uint32_t micro_begin;
     uint32_t micro_count;
@@ -192,6 +192,7 @@ struct PlanOptions {
     int min_qubits = 12;  // the state is padded to at least this many qubits
     bool mfma = false;       // SK_MFMA for dense gates of 4..5 qubits (complex64 only)
     bool mfma5 = false;      // SK_MFMA for dense gates of 5 qubits only (complex64 only)
+    bool gate_mfma = false;  // SK_MFMA for dense gates of 5 and 6 qubits, either precision
     bool mfma_fuse = false;  // also compose the gates of 5-qubit windows into SK_MFMA steps
     bool mfma_bf16 = false;  // matrix-core steps use split-bf16 products (SK_MFMA_BF16)
     int micro_bits = 4;      // register micro-steps span 3 or 4 tile bits (8 or 16 amplitudes per thread)

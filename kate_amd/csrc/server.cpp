@@ -419,6 +419,7 @@ int kate_server_create(const kate_server_options* options, kate_server** out)
     if (!err.empty()) return sfail(KATE_ERR_ARG, err);
     po.scatter = false;  // set per request, by size
     po.stream = kate::may_stream(ko, po);
+    po.gate_mfma = kate::may_gate_mfma(ko, po);
     if (po.auto_tile) {
         // one tile size, planned once per request on the scheduler thread:
         // 12-qubit tiles (a mix of 128 circuits of 12..30 qubits at

@@ -394,8 +394,8 @@ std::string plan_options(const kate_options& opt, kate::PlanOptions& po)
     po.direct = !(opt.plan_flags & KATE_PLAN_NO_DIRECT);
     po.support = !(opt.plan_flags & KATE_PLAN_NO_SUPPORT);
     // complex64: dense 5-qubit gates on the matrix cores even without
-    // use_mfma (28 qubits, 60 Haar 5-qubit gates: 62 ms against 84 ms on the
-    // VALU; 4-qubit gates stay on the register path, 24 against 31 ms)
+    // use_mfma (a simulator and a server also put 4- and 6-qubit ones there,
+    // and those of complex128: may_gate_mfma)
     po.mfma5 = opt.dtype == KATE_C64 && po.micro_bits == 4 && !(opt.plan_flags & KATE_PLAN_NO_MATRIX5);
     if (po.micro_bits != 3 && po.micro_bits != 4) return "micro_bits must be 3 or 4";
     if (po.micro_bits == 3 && opt.dtype != KATE_C128) return "micro_bits 3 needs KATE_C128";
@@ -410,6 +410,11 @@ bool may_stream(const kate_options& opt, const kate::PlanOptions& po)
 {
     return opt.tile_qubits == 0 && opt.low_qubits == 0 && opt.use_mfma == 0 && po.micro_bits == 4 && po.euler &&
            po.factor && po.direct;
+}
+
+bool may_gate_mfma(const kate_options& opt, const kate::PlanOptions& po)
+{
+    return po.micro_bits == 4 && !(opt.plan_flags & KATE_PLAN_NO_MATRIX5);
 }
 }  // namespace kate
 using kate::plan_options;
@@ -527,6 +532,7 @@ int kate_sim_create(const kate_program* program, const kate_options* options, ka
     // shapes left to the planner: streamed passes where the gates allow (the
     // device-free plan text describes the passes without them)
     po.stream = kate::may_stream(opt, po);
+    po.gate_mfma = kate::may_gate_mfma(opt, po);
     if (po.scatter) {
         // the scatter pass needs a second state buffer: only when the GPU
         // has room for both and 1 GiB to spare
