@@ -18,6 +18,7 @@
 #include <cmath>
 #include <complex>
 #include <cstring>
+#include <future>
 #include <sstream>
 
 namespace kate {
@@ -58,15 +59,17 @@ int sweep(const std::vector<uint64_t>& masks, const std::vector<uint8_t>& ok, ui
 // register op, any other is applied to the tile layout after the step; a
 // gate after a layout CNOT on one of its qubits waits for the next step.
 int sweep_micro(const std::vector<uint64_t>& masks, const std::vector<uint8_t>& ok, const std::vector<uint8_t>& lazy,
-                uint64_t set, std::vector<int>* frontier, std::vector<int>* reg, std::vector<int>* late,
-                const std::vector<uint8_t>& any = {})
+                uint64_t set, uint64_t universe, std::vector<int>* frontier, std::vector<int>* reg,
+                std::vector<int>* late, const std::vector<uint8_t>& any = {})
 {
     uint64_t blocked = 0, pending = 0;
     int count = 0;
-    for (size_t i = 0; i < masks.size(); i++) {
+    const size_t n = masks.size();
+    for (size_t i = 0; i < n; i++) {
         const uint64_t m = masks[i];
         if (m & blocked) {
             blocked |= m;
+            if (blocked == universe) break;  // no later gate can run
         } else if (lazy[i]) {
             count++;
             if ((m & ~set) == 0 && !(m & pending)) {
@@ -81,26 +84,30 @@ int sweep_micro(const std::vector<uint64_t>& masks, const std::vector<uint8_t>& 
         } else {
             if (frontier && ok[i] && !(m & pending)) frontier->push_back((int)i);
             blocked |= m;
+            if (blocked == universe) break;
         }
     }
     return count;
 }
 
 uint64_t choose_micro_set(const std::vector<uint64_t>& masks, const std::vector<uint8_t>& ok,
-                          const std::vector<uint8_t>& lazy, int width, const std::vector<uint8_t>& any = {})
+                          const std::vector<uint8_t>& lazy, int width, uint64_t universe,
+                          const std::vector<uint8_t>& any = {})
 {
     uint64_t set = 0;
+    std::vector<int> frontier;
+    std::vector<uint64_t> tried;
     for (;;) {
-        std::vector<int> frontier;
-        const int now = sweep_micro(masks, ok, lazy, set, &frontier, nullptr, nullptr, any);
+        frontier.clear();
+        const int now = sweep_micro(masks, ok, lazy, set, universe, &frontier, nullptr, nullptr, any);
         double best = 0;
         uint64_t best_new = 0;
-        std::vector<uint64_t> tried;
+        tried.clear();
         auto consider = [&](uint64_t add) {
             if (popc(set | add) > width) return;
             if (std::find(tried.begin(), tried.end(), add) != tried.end()) return;
             tried.push_back(add);
-            const int gain = sweep_micro(masks, ok, lazy, set | add, nullptr, nullptr, nullptr, any) - now;
+            const int gain = sweep_micro(masks, ok, lazy, set | add, universe, nullptr, nullptr, nullptr, any) - now;
             const double score = (double)gain / popc(add);
             if (score > best) {
                 best = score;
@@ -125,12 +132,14 @@ uint64_t choose_set(const std::vector<uint64_t>& masks, const std::vector<uint8_
                     uint64_t universe, const std::vector<uint8_t>& any = {})
 {
     uint64_t set = start;
+    std::vector<int> frontier;
+    std::vector<uint64_t> tried;
     for (;;) {
-        std::vector<int> frontier;
+        frontier.clear();
+        tried.clear();
         const int now = sweep(masks, ok, set, universe, &frontier, nullptr, any);
         double best = 0;
         uint64_t best_new = 0;
-        std::vector<uint64_t> tried;
         auto consider = [&](uint64_t add) {
             if (popc(set | add) > capacity) return;
             if (std::find(tried.begin(), tried.end(), add) != tried.end()) return;
@@ -1245,12 +1254,14 @@ struct Builder {
         while (!rem.empty()) {
             std::vector<uint64_t> tm(rem.size());
             std::vector<uint8_t> ok(rem.size()), lazy(rem.size()), any(phases ? rem.size() : 0, 0);
+            uint64_t universe = 0;
             for (size_t i = 0; i < rem.size(); i++) {
                 const PlanGate& g = prog.gates[(size_t)rem[i]];
                 uint64_t m = 0;
                 for (int j = 0; j < g.k; j++)
                     if (tile_of[g.q[j]] >= 0) m |= 1ull << tile_of[g.q[j]];
                 tm[i] = m;
+                universe |= m;
                 if (phases) any[i] = g.id == 4;
                 ok[i] = g.k <= nb && !(g.id == 0 && (opt.mfma || opt.gate_mfma) && g.k == 4);
                 lazy[i] = g.id == 3;
@@ -1294,9 +1305,9 @@ struct Builder {
                 rem.swap(next);
                 continue;
             }
-            const uint64_t set = choose_micro_set(tm, ok, lazy, nb, any);
+            const uint64_t set = choose_micro_set(tm, ok, lazy, nb, universe, any);
             std::vector<int> acc, late;
-            sweep_micro(tm, ok, lazy, set, nullptr, &acc, &late, any);
+            sweep_micro(tm, ok, lazy, set, universe, nullptr, &acc, &late, any);
             MicroStep ms{};
             std::copy(cols, cols + 16, ms.cols);
             if (acc.empty() && !late.empty()) {
@@ -2068,19 +2079,35 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
         double best = 0;
         bool have = false;
         const int lo = opt.amp_bytes == 16 && !(opt.scatter && opt.relabel) ? 2 : 3;
-        for (int low = lo; low <= lo + 3; low++) {
-            if (low > std::min(opt.tile_bits, kMaxQubits) - opt.micro_bits) break;
+        const int hi = std::min(lo + 3, std::min(opt.tile_bits, kMaxQubits) - opt.micro_bits);
+        // The candidates are independent: planned at the same time for
+        // programs whose planning (about 1 us a gate each) outweighs the
+        // start of a thread.
+        struct Cand {
+            Plan plan;
+            std::string err;
+        };
+        std::vector<std::future<Cand>> cands;
+        const auto how = opt.threads && prog.gates.size() >= 256 ? std::launch::async | std::launch::deferred
+                                                                 : std::launch::deferred;
+        for (int low = lo; low <= hi; low++) {
             o.low_qubits = low;
-            Plan cand;
-            std::string e = build_plan(prog, o, cand);
-            if (!e.empty()) {
-                if (first_err.empty()) first_err = e;
+            cands.push_back(std::async(how, [&prog, o] {
+                Cand c;
+                c.err = build_plan(prog, o, c.plan);
+                return c;
+            }));
+        }
+        for (std::future<Cand>& f : cands) {
+            Cand c = f.get();
+            if (!c.err.empty()) {
+                if (first_err.empty()) first_err = c.err;
                 continue;
             }
-            const double cost = plan_cost(cand, opt.amp_bytes);
+            const double cost = plan_cost(c.plan, opt.amp_bytes);
             if (!have || cost < best) {
                 best = cost;
-                plan = std::move(cand);
+                plan = std::move(c.plan);
                 have = true;
             }
         }
