@@ -1861,9 +1861,33 @@ static uint64_t permute_bits(const std::vector<int>& to, uint64_t x)
     return y;
 }
 
+// Tile numbers of an out-of-place pass: neighbouring workgroups run on the
+// eight XCDs in turn, each with its own L2, so the rest qubits written to the
+// lowest offsets become bits 3 and up of the tile number and the highest ones
+// bits 0..2.  Tiles that write parts of one line then follow each other on
+// one XCD and the parts leave its L2 together (30-qubit layered circuit,
+// complex128: 16 passes with 32 B runs 220 -> 151 ms, 19 with 64 B runs
+// 152.3 -> 150.5; runs of whole lines are as fast either way).
+static void order_writes(PassArgs& pa, ScatterArgs& sa)
+{
+    constexpr int kXcdBits = 3;
+    if (pa.nrest <= kXcdBits) return;
+    std::vector<int> by((size_t)pa.nrest);
+    for (int i = 0; i < pa.nrest; i++) by[(size_t)i] = i;
+    std::stable_sort(by.begin(), by.end(),
+                     [&](int a, int b) { return __builtin_ctzll(sa.out_rest[a]) < __builtin_ctzll(sa.out_rest[b]); });
+    std::rotate(by.begin(), by.end() - kXcdBits, by.end());
+    const PassArgs pf = pa;
+    const ScatterArgs sf = sa;
+    for (int i = 0; i < pa.nrest; i++) {
+        pa.rest_pos[i] = pf.rest_pos[by[(size_t)i]];
+        sa.out_rest[i] = sf.out_rest[by[(size_t)i]];
+    }
+}
+
 static void make_relabel(Plan& plan)
 {
-    const int n = plan.nq_int, t = plan.tile_bits;
+    const int n = plan.nq_int, t = plan.tile_bits, low = std::min(plan.low_qubits, t);
     const size_t np = plan.passes.size();
     if (n > 64 || plan.remap_passes || np < 3 || plan.pass_zero.size() < np) return;
     size_t start = np;
@@ -1890,7 +1914,15 @@ static void make_relabel(Plan& plan)
         PassArgs& pa = plan.passes[k];
         if (k + 1 < np) {
             const PassArgs& nx = plan.passes[k + 1];
-            for (int b = 0; b < t; b++) Q[nx.load_pos[b]] = b;
+            // The next tile's low qubits, then those this tile holds too, at
+            // the lowest offsets: a write run is 2^(low + shared) amplitudes.
+            uint64_t here = 0;
+            for (int b = 0; b < t; b++) here |= 1ull << pa.store_pos[b];
+            int at = 0;
+            for (int b = 0; b < low; b++) Q[nx.load_pos[b]] = at++;
+            for (uint64_t shared : {1ull, 0ull})
+                for (int b = low; b < t; b++)
+                    if (((here >> nx.load_pos[b]) & 1ull) == shared) Q[nx.load_pos[b]] = at++;
             for (int i = 0; i < nx.nrest; i++) Q[nx.rest_pos[i]] = t + i;
         } else {
             for (int q = 0; q < n; q++) Q[(size_t)q] = q;
@@ -1919,6 +1951,7 @@ static void make_relabel(Plan& plan)
         for (int b = 0; b < t; b++) pa.load_pos[b] = (uint8_t)P[pa.load_pos[b]];
         for (int i = 0; i < pa.nrest; i++) pa.rest_pos[i] = (uint8_t)P[pa.rest_pos[i]];
         for (int i = 0; i < 16; i++) pa.first_g[i] = permute_bits(P, pa.first_g[i]);
+        order_writes(pa, plan.scatter_args[pa.scatter_idx]);
         P = Q;
     }
     plan.support_passes = std::min(plan.support_passes, (int)start);
@@ -2068,17 +2101,15 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
         // relabelled passes the reads are whole blocks whatever the low
         // qubits, so plans with fewer low qubits and fewer passes gain
         // (30-qubit layered circuit, complex64 13-qubit tiles: 18 passes with
-        // 3 low qubits 85.6 ms, 25 with 5 96.6 ms).  Relabelled complex128
-        // plans keep at least 3 low qubits (128 B runs): with 2 the same
-        // circuit takes 19 passes and 158 ms against 24 passes and 162 ms,
-        // but each pass moves its 34.4 GB in 10.2 ms instead of 7.9 ms; the
-        // longer runs are kept for the passes' nearness to their HBM bound.
+        // 3 low qubits 85.6 ms, 25 with 5 96.6 ms; complex128: 19 passes with
+        // 2 low qubits 150.5 ms, 24 with 3 157.6 ms, both bound by their
+        // register steps more than by their lines).
         PlanOptions o = opt;
         o.auto_low = false;
         std::string first_err;
         double best = 0;
         bool have = false;
-        const int lo = opt.amp_bytes == 16 && !(opt.scatter && opt.relabel) ? 2 : 3;
+        const int lo = opt.amp_bytes == 16 ? 2 : 3;
         const int hi = std::min(lo + 3, std::min(opt.tile_bits, kMaxQubits) - opt.micro_bits);
         // The candidates are independent: planned at the same time for
         // programs whose planning (about 1 us a gate each) outweighs the
