@@ -1389,10 +1389,15 @@ int stream_r(int tile_bits, void* state, const PassArgs& pa, const DevPlan& dp, 
     if (pa.micro_bits != 4 || (pa.scatter && (!dp.dst || !dp.scatter)) || pa.phase_count > kTilePhases ||
         (pa.phase_count && !dp.phases))
         return (int)hipErrorInvalidValue;
-    // the planner streams only plans whose tile size it chose: 12 qubits, or 13
-    // for complex64 plans of light passes, whose permutations stay off k_stream
-    if (tile_bits != 12) return (int)hipErrorInvalidValue;
-    return stream_t<R, 12>(state, pa, dp, s);
+    // the planner streams only plans whose tile size it chose: 12 qubits, 10 or
+    // 11 for states that small, 13 for complex64 plans of light passes, whose
+    // permutations stay off k_stream
+    switch (tile_bits) {
+    case 10: return stream_t<R, 10>(state, pa, dp, s);
+    case 11: return stream_t<R, 11>(state, pa, dp, s);
+    case 12: return stream_t<R, 12>(state, pa, dp, s);
+    default: return (int)hipErrorInvalidValue;
+    }
 }
 
 // ---- many circuits in one persistent launch ---------------------------------

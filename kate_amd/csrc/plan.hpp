@@ -104,8 +104,8 @@ constexpr int kMaxQubits = 40;
 
 // One pass over the state: tile bit b of the LDS tile is state qubit
 // load_pos[b] when the tile is read and store_pos[b] when it is written back
-// (they differ only for qubit remaps).  rest_pos lists the other qubits in
-// ascending order; block index bit i is qubit rest_pos[i].
+// (they differ only for qubit remaps).  rest_pos lists the other qubits, in
+// ascending order in place; tile number bit i is qubit rest_pos[i].
 struct PassArgs {
     uint8_t tile_bits;
     uint8_t nrest;

@@ -300,6 +300,7 @@ void plan_request(const kate_server* s, Request& r)
     // tile blocks
     kate::PlanOptions po = s->po;
     po.scatter = r.prog.nqubits >= kServeOutOfPlaceQubits;
+    kate::fit_tile(s->opt.tile_qubits, s->opt.low_qubits, r.prog.nqubits, po);
     // a product-state input has no support region to follow: its passes can
     // all be relabelled
     po.zero_start = r.theta_phi.empty();
