@@ -202,6 +202,12 @@ int kate_batch_create(const kate_program* programs, int32_t count, const kate_op
         for (size_t i = 0; i < plan.passes.size(); i++) {
             kate::PassArgs pa = plan.passes[i];
             pa.micro_begin += mb;
+            pa.ops_begin += ob;
+            pa.ops_end += ob;
+            pa.coef_begin += cb;
+            pa.coef_end += cb;
+            pa.raw_begin += rb;
+            pa.raw_end += rb;
             passes.push_back(pa);
             pass_zero.push_back(i < plan.pass_zero.size() && (int)i < plan.support_passes ? plan.pass_zero[i] : 0ull);
         }

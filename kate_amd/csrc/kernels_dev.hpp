@@ -941,7 +941,61 @@ __device__ __forceinline__ void scatter_store(Cx<R>* __restrict__ dst, const Pas
     }
 }
 
-template <typename R, int TB, int WIDE, int NB, bool LIGHT>
+// A step is a chain of scalar loads: its descriptor, its ops, their coefficients.
+// After a kernel boundary (a fence, in a batch) they miss the XCD's L2, and a
+// workgroup that shares its CU with at most one other waits for each, so the
+// passes of small states and of batches (WARM) fetch what they read of the plan
+// into L2 under the loads of the amplitudes, one vector load a line (20
+// qubits, 10 layers, complex128: a call 260 -> 231 us; 256 complex64 circuits of
+// 10-20 qubits 3.14 -> 3.07 ms).  Reading the lines into the scalar cache as well
+// gained nothing there (234 us) and cost a pass of one tile 11 us.
+constexpr uint32_t kWarmLine = 128;
+
+// Starts fetching the first WL * NT lines of what the pass reads of the
+// plan's pools into L2 and returns the words read: the caller consumes them
+// (warm_done) once its amplitudes are on their way.
+template <typename R, int NT, int WL>
+__device__ __forceinline__ void warm_plan(const PassArgs& pa, const MicroStep* __restrict__ micro,
+                                          const MicroOp* __restrict__ ops, const Cx<R>* __restrict__ coef,
+                                          const uint32_t* __restrict__ raw, uint32_t (&x)[WL])
+{
+    // every pool starts at a line and holds whole words: the line of a word
+    // of a range starts inside the pool
+    const char* base[4] = {reinterpret_cast<const char*>(micro), reinterpret_cast<const char*>(coef),
+                           reinterpret_cast<const char*>(ops), reinterpret_cast<const char*>(raw)};
+    const uint64_t begin[4] = {(uint64_t)pa.micro_begin * sizeof(MicroStep), (uint64_t)pa.coef_begin * sizeof(Cx<R>),
+                               (uint64_t)pa.ops_begin * sizeof(MicroOp), (uint64_t)pa.raw_begin * 4u};
+    const uint64_t end[4] = {(uint64_t)(pa.micro_begin + pa.micro_count) * sizeof(MicroStep),
+                             (uint64_t)pa.coef_end * sizeof(Cx<R>), (uint64_t)pa.ops_end * sizeof(MicroOp),
+                             (uint64_t)pa.raw_end * 4u};
+    uint32_t total = 0, first[4];
+    uint64_t from[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        first[r] = total;
+        from[r] = begin[r] / kWarmLine;
+        if (end[r] > begin[r]) total += (uint32_t)((end[r] - 1) / kWarmLine - from[r]) + 1u;
+    }
+#pragma unroll
+    for (int i = 0; i < WL; i++) {
+        // (micro_count > 0: at least one line)
+        const uint32_t want = threadIdx.x + (uint32_t)(i * NT), l = want < total ? want : total - 1u;
+        const char* p = base[0] + kWarmLine * (from[0] + l);
+#pragma unroll
+        for (int r = 1; r < 4; r++)
+            if (l >= first[r]) p = base[r] + kWarmLine * (from[r] + (l - first[r]));
+        x[i] = *reinterpret_cast<const uint32_t*>(p);
+    }
+}
+
+template <int WL>
+__device__ __forceinline__ void warm_done(const uint32_t (&x)[WL])
+{
+#pragma unroll
+    for (int i = 0; i < WL; i++) asm volatile("" ::"v"(x[i]));
+}
+
+template <typename R, int TB, int WIDE, int NB, bool LIGHT, bool WARM>
 __device__ __forceinline__ void tile_pass(Cx<R>* __restrict__ state, const PassArgs& pa, uint64_t blk, Cx<R>* tile,
                                           const MicroStep* __restrict__ micro, const MicroOp* __restrict__ ops,
                                           const Cx<R>* __restrict__ coef, const uint32_t* __restrict__ raw,
@@ -953,6 +1007,10 @@ __device__ __forceinline__ void tile_pass(Cx<R>* __restrict__ state, const PassA
 
     const uint64_t base = rest_base(pa, blk);
     uint32_t m_begin = 0, m_end = pa.micro_count;
+    constexpr int WL = NT < 128 ? 2 : 1;
+    uint32_t warm[WL] = {};
+    if constexpr (WARM)
+        if (pa.micro_count) warm_plan<R, NT, WL>(pa, micro, ops, coef, raw, warm);
 
     if (pa.fuse_first) {
         // direct first step: HBM -> registers -> ops -> LDS in the step's layout
@@ -971,6 +1029,7 @@ __device__ __forceinline__ void tile_pass(Cx<R>* __restrict__ state, const PassA
 #pragma unroll
             for (int s = 0; s < N; s++) v[s] = state[gt ^ direct_reg_offset<NB>(pa.first_g, s)];
         }
+        if constexpr (WARM) warm_done(warm);
         const uint32_t f = reg_step_ops<R, N, LIGHT>(v, msp, op_begin, op_count, ops, coef);
         m_begin = 1;
         if (pa.micro_count == 1 && pa.fuse_last) {
@@ -1026,6 +1085,7 @@ __device__ __forceinline__ void tile_pass(Cx<R>* __restrict__ state, const PassA
                 r[i] = state[off];
             }
         }
+        if constexpr (WARM) warm_done(warm);
         const uint32_t tsw = swz<R>(tid) * (uint32_t)sizeof(Cx<R>);
 #pragma unroll
         for (int i = 0; i < N; i++) lds_at(tile, tsw ^ (swz<R>((uint32_t)i * NT) * (uint32_t)sizeof(Cx<R>))) = r[i];
@@ -1074,7 +1134,7 @@ constexpr int kPassWavesPerEU =
                                          : 1);
 
 // LIGHT: the pass's ops are all in the light set (apply_op_light).
-template <typename R, int TB, int WIDE, int NB, bool LIGHT>
+template <typename R, int TB, int WIDE, int NB, bool LIGHT, bool WARM = false>
 __global__ __launch_bounds__(1 << (TB - NB)) __attribute__((amdgpu_waves_per_eu(kPassWavesPerEU<R, TB, WIDE, NB, LIGHT>)))
 void k_pass(Cx<R>* __restrict__ state, PassArgs pa,
                                                          const MicroStep* __restrict__ micro,
@@ -1085,7 +1145,7 @@ void k_pass(Cx<R>* __restrict__ state, PassArgs pa,
                                                          const ScatterArgs* __restrict__ sa)
 {
     __shared__ Cx<R> tile[1 << TB];
-    tile_pass<R, TB, WIDE, NB, LIGHT>(state, pa, blockIdx.x, tile, micro, ops, coef, raw, dst, sa);
+    tile_pass<R, TB, WIDE, NB, LIGHT, WARM>(state, pa, blockIdx.x, tile, micro, ops, coef, raw, dst, sa);
 }
 
 // ---- streamed passes -----------------------------------------------------------
@@ -1240,7 +1300,7 @@ __device__ __forceinline__ StreamStep load_stream_step(const MicroStep* __restri
 template <typename R, int TB>
 constexpr int kStreamWavesPerEU = kLdsWavesPerSimd<R, TB, 4> > 4 ? 4 : kLdsWavesPerSimd<R, TB, 4>;
 
-template <typename R, int TB>
+template <typename R, int TB, bool WARM>
 __global__ __launch_bounds__(1 << (TB - 4)) __attribute__((amdgpu_waves_per_eu(kStreamWavesPerEU<R, TB>)))
 void k_stream(const Cx<R>* state, PassArgs pa, const MicroStep* __restrict__ micro,
               const uint32_t* __restrict__ codes, const Phase* __restrict__ phases,
@@ -1252,6 +1312,10 @@ void k_stream(const Cx<R>* state, PassArgs pa, const MicroStep* __restrict__ mic
     const uint32_t tid = threadIdx.x;
     const uint64_t blk = blockIdx.x, base = rest_base(pa, blk);
     const MicroStep* __restrict__ ms = micro + pa.micro_begin;
+    constexpr int WL = NT < 128 ? 2 : 1;
+    uint32_t warm[WL] = {};
+    if constexpr (WARM)
+        if (pa.micro_count) warm_plan<R, NT, WL>(pa, micro, (const MicroOp*)codes, coef, codes, warm);
     Cx<R> v[N];
     {
         // the first step's amplitudes straight into its registers, or the
@@ -1286,6 +1350,7 @@ void k_stream(const Cx<R>* state, PassArgs pa, const MicroStep* __restrict__ mic
             for (int s = 0; s < N; s++) v[s] = state[offset(s)];
         }
     }
+    if constexpr (WARM) warm_done(warm);
     // the tile's factors of the pass's phases, one thread each, while the
     // amplitudes come in
     for (uint32_t p = tid; p < pa.phase_count; p += NT) {
@@ -1375,15 +1440,15 @@ void k_stream(const Cx<R>* state, PassArgs pa, const MicroStep* __restrict__ mic
     }
 }
 
-template <typename R, int TB>
+template <typename R, int TB, bool WARM>
 int stream_t(void* state, const PassArgs& pa, const DevPlan& dp, hipStream_t s)
 {
-    hipLaunchKernelGGL((k_stream<R, TB>), dim3(1u << pa.nrest), dim3(1 << (TB - 4)), 0, s, (const Cx<R>*)state, pa,
+    hipLaunchKernelGGL((k_stream<R, TB, WARM>), dim3(1u << pa.nrest), dim3(1 << (TB - 4)), 0, s, (const Cx<R>*)state, pa,
                        dp.micro, dp.raw, dp.phases, (const Cx<R>*)dp.coef, (Cx<R>*)(pa.scatter ? dp.dst : state), dp.scatter);
     return (int)hipGetLastError();
 }
 
-template <typename R>
+template <typename R, bool WARM>
 int stream_r(int tile_bits, void* state, const PassArgs& pa, const DevPlan& dp, hipStream_t s)
 {
     if (pa.micro_bits != 4 || (pa.scatter && (!dp.dst || !dp.scatter)) || pa.phase_count > kTilePhases ||
@@ -1393,9 +1458,9 @@ int stream_r(int tile_bits, void* state, const PassArgs& pa, const DevPlan& dp, 
     // 11 for states that small, 13 for complex64 plans of light passes, whose
     // permutations stay off k_stream
     switch (tile_bits) {
-    case 10: return stream_t<R, 10>(state, pa, dp, s);
-    case 11: return stream_t<R, 11>(state, pa, dp, s);
-    case 12: return stream_t<R, 12>(state, pa, dp, s);
+    case 10: return stream_t<R, 10, WARM>(state, pa, dp, s);
+    case 11: return stream_t<R, 11, WARM>(state, pa, dp, s);
+    case 12: return stream_t<R, 12, WARM>(state, pa, dp, s);
     default: return (int)hipErrorInvalidValue;
     }
 }
@@ -1473,7 +1538,7 @@ void k_batch(Cx<R>* __restrict__ states,
             }
             __syncthreads();
         }
-        tile_pass<R, TB, WIDE, NB, false>(states + circ_off[task.circuit], passes[task.pass], task.tile, tile, micro, ops,
+        tile_pass<R, TB, WIDE, NB, false, true>(states + circ_off[task.circuit], passes[task.pass], task.tile, tile, micro, ops,
                                           coef, raw, nullptr, nullptr);
         // every wave's stores of this tile have completed (each wave drains
         // its memory counters; a workgroup-scope barrier alone does not wait
@@ -1530,6 +1595,34 @@ int pass_r(int tile_bits, void* state, int nq_int, const PassArgs& pa, const Dev
     case 11: return pass_nb<R, 11>(state, nq_int, pa, dp, s);
     case 12: return pass_nb<R, 12>(state, nq_int, pa, dp, s);
     case 13: return pass_nb<R, 13>(state, nq_int, pa, dp, s);
+    default: return (int)hipErrorInvalidValue;
+    }
+}
+
+// Passes of register steps with 16 amplitudes per thread, the plan fetched
+// ahead.
+template <typename R, int TB>
+int warm_t(void* state, const PassArgs& pa, const DevPlan& dp, hipStream_t s)
+{
+    const dim3 grid(1u << pa.nrest), block(1 << (TB - 4));
+    if (pa.light)
+        hipLaunchKernelGGL((k_pass<R, TB, kRegSteps, 4, true, true>), grid, block, 0, s, (Cx<R>*)state, pa,
+                           dp.micro, dp.ops, (const Cx<R>*)dp.coef, dp.raw, (Cx<R>*)dp.dst, dp.scatter);
+    else
+        hipLaunchKernelGGL((k_pass<R, TB, kRegSteps, 4, false, true>), grid, block, 0, s, (Cx<R>*)state, pa,
+                           dp.micro, dp.ops, (const Cx<R>*)dp.coef, dp.raw, (Cx<R>*)dp.dst, dp.scatter);
+    return (int)hipGetLastError();
+}
+
+template <typename R>
+int warm_r(int tile_bits, void* state, const PassArgs& pa, const DevPlan& dp, hipStream_t s)
+{
+    if (pa.stream) return stream_r<R, true>(tile_bits, state, pa, dp, s);
+    switch (tile_bits) {
+    case 10: return warm_t<R, 10>(state, pa, dp, s);
+    case 11: return warm_t<R, 11>(state, pa, dp, s);
+    case 12: return warm_t<R, 12>(state, pa, dp, s);
+    case 13: return warm_t<R, 13>(state, pa, dp, s);
     default: return (int)hipErrorInvalidValue;
     }
 }

@@ -1205,6 +1205,18 @@ struct Builder {
     // QFT: 14 passes, 5.05 ms; streamed with phases 3 passes, 1.33 ms).
     std::string pack_micro(const std::vector<int>& gl, const int* tile_of, PassArgs& pa)
     {
+        pa.ops_begin = (uint32_t)plan.ops.size();
+        pa.coef_begin = (uint32_t)(plan.coef.size() / 2);
+        pa.raw_begin = (uint32_t)plan.raw.size();
+        const std::string e = pack_micro_form(gl, tile_of, pa);
+        pa.ops_end = (uint32_t)plan.ops.size();
+        pa.coef_end = (uint32_t)(plan.coef.size() / 2);
+        pa.raw_end = (uint32_t)plan.raw.size();
+        return e;
+    }
+
+    std::string pack_micro_form(const std::vector<int>& gl, const int* tile_of, PassArgs& pa)
+    {
         if (opt.stream && opt.micro_bits == 4) {
             bool all = true;
             for (int g : gl) all = all && streamable(prog.gates[(size_t)g]);
@@ -1572,7 +1584,7 @@ struct Builder {
             pa.micro_begin = (uint32_t)plan.micro.size();
             pa.micro_count = 0;
             for (int b = 0; b < 16; b++) pa.store_cols[b] = (uint16_t)(1u << b);
-                fill_store_bytes(pa);
+            fill_store_bytes(pa);
             // a remap pass writes every tile (masked reads of the zero
             // qubits); the support is not tracked through it
             plan.pass_zero.push_back(remapped ? 0ull : zero);

@@ -152,6 +152,8 @@ struct PassArgs {
     uint32_t phase_begin;  // streamed: its phases in Plan::phases
     uint32_t phase_count;
     uint64_t last_xor;  // streamed direct last step: XORed into every stored offset
+    // What the pass reads of the plan's pools beside its micro-steps, [begin, end).
+    uint32_t ops_begin, ops_end, coef_begin, coef_end, raw_begin, raw_end;
 };
 
 // Store side of a scatter pass: store index bit k of a tile goes to state

@@ -6,7 +6,7 @@ namespace kate {
 
 int launch_stream_f32(int tile_bits, void* state, const PassArgs& pa, const DevPlan& dp, void* stream)
 {
-    return stream_r<float>(tile_bits, state, pa, dp, (hipStream_t)stream);
+    return stream_r<float, false>(tile_bits, state, pa, dp, (hipStream_t)stream);
 }
 
 }  // namespace kate
