@@ -340,7 +340,7 @@ int kate_batch_last_ms(const kate_batch* batch, float* ms);
 
 /* ---- serving: continuous batching of simulate requests ----
  * No counterpart in Kate.  One HBM arena reserved at creation (no allocation
- * while serving), a pool of streams and one scheduler thread: requests are
+ * while serving), a pool of streams, planner threads and one scheduler thread: requests are
  * planned off the caller's thread, admitted first come first served as soon
  * as their footprint fits the free arena, and run on the stream pool so that
  * requests in flight overlap on the device.  Each returns <Z_S> for up to 15
