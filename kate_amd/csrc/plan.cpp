@@ -1196,13 +1196,14 @@ struct Builder {
     }
 
     // Packs the gates of one pass (`gl`, program order) into micro-steps:
-    // streamed if they all allow it and the light kernel does not, else as
-    // register ops and wide steps.  Light passes (30-qubit layered circuit,
-    // complex128: 6.9 ms a sweep pass, 13.0 ms a pass that mixes CNOTs and
-    // rotations; 28 qubits complex64, 13-qubit tiles: 1.2 and 2.2-2.6 ms) run
-    // 5 % slower streamed (7.4, 13.3; 1.2, 2.3-2.7); passes of CRk gates run
-    // several times faster, most of all because far fewer remain (25-qubit
-    // QFT: 14 passes, 5.05 ms; streamed with phases 3 passes, 1.33 ms).
+    // streamed in programs with CRk gates (`phases`), whose passes run several
+    // times faster so, most of all because far fewer remain (25-qubit QFT
+    // complex128: 14 passes, 5.05 ms; streamed 3 passes, 1.33 ms), else as
+    // register ops and wide steps.  Without CRk the register ops are the faster
+    // form: light passes run 5 % slower streamed (30-qubit layered circuit,
+    // complex128: 6.9 and 7.4 ms a sweep pass), passes of Hadamards and CNOTs
+    // 15-20 % (QulacsBench, complex128: 28 qubits 51.5 and 62.9 ms, 25 qubits
+    // 6.4 and 7.4 ms; 22 qubits 0.99 and 0.97).
     std::string pack_micro(const std::vector<int>& gl, const int* tile_of, PassArgs& pa)
     {
         pa.ops_begin = (uint32_t)plan.ops.size();
@@ -1217,33 +1218,13 @@ struct Builder {
 
     std::string pack_micro_form(const std::vector<int>& gl, const int* tile_of, PassArgs& pa)
     {
-        if (opt.stream && opt.micro_bits == 4) {
-            bool all = true;
-            for (int g : gl) all = all && streamable(prog.gates[(size_t)g]);
-            if (all) {
-                const size_t nm = plan.micro.size(), no = plan.ops.size(), nc = plan.coef.size(), nr = plan.raw.size(),
-                             np = plan.phases.size();
-                auto undo = [&] {
-                    plan.phases.resize(np);
-                    plan.micro.resize(nm);
-                    plan.ops.resize(no);
-                    plan.coef.resize(nc);
-                    plan.raw.resize(nr);
-                };
-                // passes of the light set stay on the light kernel
-                std::string e = phases ? "phases" : pack_micro_as(gl, tile_of, pa);
-                if (e.empty() && pa.light) return "";
-                undo();
-                pa.stream = 1;
-                phase_begin = pa.phase_begin = (uint32_t)np;
-                e = pack_micro_as(gl, tile_of, pa);
-                pa.phase_count = (uint32_t)(plan.phases.size() - np);
-                if (pa.phase_count > kTilePhases) e = "not streamable";
-                if (e != "not streamable" || phases) return e;
-                undo();
-                pa.stream = 0;
-                pa.phase_count = 0;
-            }
+        if (phases) {
+            const size_t np = plan.phases.size();
+            pa.stream = 1;
+            phase_begin = pa.phase_begin = (uint32_t)np;
+            const std::string e = pack_micro_as(gl, tile_of, pa);
+            pa.phase_count = (uint32_t)(plan.phases.size() - np);
+            return e.empty() && pa.phase_count > kTilePhases ? "not streamable" : e;
         }
         return pack_micro_as(gl, tile_of, pa);
     }
