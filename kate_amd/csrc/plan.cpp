@@ -247,7 +247,8 @@ bool kron_factors(const double* m, double (&a)[8], double (&b)[8])
         for (int j = 0; j < 4; j++) {
             const double re = a[2 * i] * b[2 * j] - a[2 * i + 1] * b[2 * j + 1];
             const double im = a[2 * i] * b[2 * j + 1] + a[2 * i + 1] * b[2 * j];
-            if (std::fabs(re - R[i][j][0]) > 2e-15 || std::fabs(im - R[i][j][1]) > 2e-15) return false;
+            // (a NaN entry fails this too, and the gate stays whole)
+            if (!(std::fabs(re - R[i][j][0]) <= 2e-15 && std::fabs(im - R[i][j][1]) <= 2e-15)) return false;
         }
     return true;
 }
@@ -740,6 +741,9 @@ struct Builder {
         h.count++;
     }
 
+    // An entry of a gate's Euler form equals the gate's to rounding; false for NaN.
+    static bool near(std::complex<double> a, std::complex<double> b) { return std::abs(a - b) <= 1e-14; }
+
     // Euler form of a 2x2 unitary u (row-major, interleaved):
     // u = diag(p0, p1) * [[x, -iy], [-iy, x]] * diag(1, q) with x = |u00| and
     // y real.  q is set to exactly 1 (has_q false) when it differs from 1 by at
@@ -767,9 +771,7 @@ struct Builder {
         }
         p[1] = I * u10 / y;  // u10 = -i p1 y
         const cd r00 = p[0] * x, r01 = -I * p[0] * y * q, r10 = -I * p[1] * y, r11 = p[1] * x * q;
-        const double err = std::max(std::max(std::abs(r00 - u00), std::abs(r01 - u01)),
-                                    std::max(std::abs(r10 - u10), std::abs(r11 - u11)));
-        return err <= 1e-14;
+        return near(r00, u00) && near(r01, u01) && near(r10, u10) && near(r11, u11);
     }
 
     // The held dense gates of the micro bits in `kron` as one Euler-form
@@ -932,8 +934,7 @@ struct Builder {
             return false;
         }
         const cd r00 = p[0] * x, r01 = -I * p[0] * y * q, r10 = -I * p[1] * y, r11 = p[1] * x * q;
-        return std::max(std::max(std::abs(r00 - u00), std::abs(r01 - u01)),
-                        std::max(std::abs(r10 - u10), std::abs(r11 - u11))) <= 1e-14;
+        return near(r00, u00) && near(r01, u01) && near(r10, u10) && near(r11, u11);
     }
 
     // One register step as a stream of rotations and diagonals.  Register s
