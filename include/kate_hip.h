@@ -270,7 +270,8 @@ int kate_sim_execute_timed(kate_sim* sim, const double* theta_phi_in, double* th
 /* Pass plan as text (one line per pass), for inspection and tests. */
 int kate_sim_describe(kate_sim* sim, char* buf, size_t len);
 /* The same plan without a device (no counterpart in Kate, whose grouping is
- * fixed by gateGrouping): pass and remap counts plus the text form. */
+ * fixed by gateGrouping): pass and remap counts plus the text form.  Equal to
+ * the simulator's wherever the GPU has room for a second state buffer. */
 int kate_plan_describe(const kate_program* program, const kate_options* options, int32_t* passes,
                        int32_t* remap_passes, char* buf, size_t len);
 

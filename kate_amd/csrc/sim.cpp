@@ -421,7 +421,8 @@ bool may_gate_mfma(const kate_options& opt, const kate::PlanOptions& po)
 // workgroup, bound by the latency of one register step after the other, and a
 // step on a quarter of the amplitudes is shorter (10 qubits, 10 layers: 23
 // steps in 59 us with the 12-qubit tile, 46 us with 10; complex64 50 and 43 us).
-// The buffer stays 4096 amplitudes long; tiles past the state are not run.
+// The buffer stays 4096 amplitudes long; only the last pass runs its tiles past
+// the state (it writes their zeros).
 void fit_tile(int tile_qubits, int low_qubits, int nqubits, kate::PlanOptions& po)
 {
     if (tile_qubits || low_qubits || nqubits >= 12) return;
@@ -431,6 +432,28 @@ void fit_tile(int tile_qubits, int low_qubits, int nqubits, kate::PlanOptions& p
 }
 }  // namespace kate
 using kate::plan_options;
+
+namespace {
+
+// A simulator's plan of a program (sim_options, then sim_plan): the one that
+// kate_sim_create runs and kate_plan_describe describes.  Only whether the GPU
+// has room for a second state buffer (PlanOptions::scatter) is left to the
+// creation.
+std::string sim_options(const kate_options& opt, kate::PlanOptions& po)
+{
+    std::string err = plan_options(opt, po);
+    po.stream = kate::may_stream(opt, po);
+    po.gate_mfma = kate::may_gate_mfma(opt, po);
+    return err;
+}
+
+std::string sim_plan(const kate_options& opt, const kate::Program& prog, kate::PlanOptions& po, kate::Plan& plan)
+{
+    kate::fit_tile(opt.tile_qubits, opt.low_qubits, prog.nqubits, po);
+    return kate::build_plan(prog, po, plan);
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -493,13 +516,13 @@ int kate_plan_describe(const kate_program* program, const kate_options* options,
     kate_options opt{};
     if (options) opt = *options;
     kate::PlanOptions po;
-    std::string err = plan_options(opt, po);
+    std::string err = sim_options(opt, po);
     if (!err.empty()) return fail(KATE_ERR_ARG, err);
     kate::Program prog;
     err = to_program(program, prog);
     if (!err.empty()) return fail(KATE_ERR_PROGRAM, err);
     kate::Plan plan;
-    err = kate::build_plan(prog, po, plan);
+    err = sim_plan(opt, prog, po, plan);
     if (!err.empty()) return fail(KATE_ERR_PROGRAM, "planning: " + err);
     if (passes) *passes = plan.gate_passes;
     if (remap_passes) *remap_passes = plan.remap_passes;
@@ -535,18 +558,13 @@ int kate_sim_create(const kate_program* program, const kate_options* options, ka
         return fail(KATE_ERR_PROGRAM, err);
     }
     kate::PlanOptions po;
-    err = plan_options(opt, po);
+    err = sim_options(opt, po);
     if (!err.empty()) {
         delete s;
         return fail(KATE_ERR_ARG, err);
     }
     s->support = po.support;
     s->defer = po.defer;
-    // shapes left to the planner: streamed passes where the gates allow (the
-    // device-free plan text describes the passes without them)
-    po.stream = kate::may_stream(opt, po);
-    po.gate_mfma = kate::may_gate_mfma(opt, po);
-    kate::fit_tile(opt.tile_qubits, opt.low_qubits, s->prog.nqubits, po);
     if (po.scatter) {
         // the scatter pass needs a second state buffer: only when the GPU
         // has room for both and 1 GiB to spare
@@ -557,7 +575,7 @@ int kate_sim_create(const kate_program* program, const kate_options* options, ka
             (unsigned __int128)fr < need)
             po.scatter = false;
     }
-    err = kate::build_plan(s->prog, po, s->plan);
+    err = sim_plan(opt, s->prog, po, s->plan);
     if (!err.empty()) {
         delete s;
         return fail(KATE_ERR_PROGRAM, "planning: " + err);
