@@ -1150,7 +1150,8 @@ void k_pass(Cx<R>* __restrict__ state, PassArgs pa,
 
 // ---- streamed passes -----------------------------------------------------------
 //
-// k_stream runs the passes of 1-qubit, CNOT and CRk gates (PassArgs::stream).
+// k_stream runs the passes of programs of 1-qubit, CNOT and CRk gates whose CRk
+// gates make it the cheaper form (PassArgs::stream; the planner's streams_pay).
 // Each register step is a stream of three ops -- a rotation along any register
 // direction, a 16-entry diagonal, a phase of the thread -- and writes its
 // registers back through a linear map, so CNOTs inside a step cost nothing

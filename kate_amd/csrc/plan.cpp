@@ -1114,10 +1114,16 @@ struct Builder {
         return true;
     }
 
-    // Gates a streamed pass can run.
-    bool streamable(const PlanGate& g) const
+    // Whether a program's passes can be streamed: 1-qubit, CNOT and CRk gates,
+    // CRk among them.
+    static bool streamable(const Program& prog)
     {
-        return g.id == 2 || g.id == 3 || g.id == 4 || (g.id == 0 && g.k == 1);
+        bool crk = false;
+        for (const PlanGate& g : prog.gates) {
+            if (!(g.id == 2 || g.id == 3 || g.id == 4 || (g.id == 0 && g.k == 1))) return false;
+            crk = crk || g.id == 4;
+        }
+        return crk;
     }
 
     // The gates `acc` of a register step as a stream in `ms`.
@@ -1197,8 +1203,8 @@ struct Builder {
     }
 
     // Packs the gates of one pass (`gl`, program order) into micro-steps:
-    // streamed in programs with CRk gates (`phases`), whose passes run several
-    // times faster so, most of all because far fewer remain (25-qubit QFT
+    // streamed in programs whose CRk gates make that the cheaper form (`phases`,
+    // streams_pay), most of all because far fewer passes remain (25-qubit QFT
     // complex128: 14 passes, 5.05 ms; streamed 3 passes, 1.33 ms), else as
     // register ops and wide steps.  Without CRk the register ops are the faster
     // form: light passes run 5 % slower streamed (30-qubit layered circuit,
@@ -2015,6 +2021,23 @@ static double relabel_run_cost(int run_bytes)
     return run_bytes <= 32 ? 2.5 : 0.6;
 }
 
+// The fraction of pass i's tiles that a run from |0...0> launches.
+static double launched(const Plan& p, size_t i)
+{
+    double f = 1.0;
+    if ((int)i < p.support_passes && i < p.pass_zero.size())
+        for (int j = 0; j < p.passes[i].nrest; j++)
+            if ((p.pass_zero[i] >> p.passes[i].rest_pos[j]) & 1ull) f *= 0.5;
+    return f;
+}
+
+// How the candidate plans of a program are planned: at the same time where their
+// planning (about 1 us a gate each) outweighs the start of a thread.
+static std::launch plan_launch(const Program& prog, const PlanOptions& opt)
+{
+    return opt.threads && prog.gates.size() >= 256 ? std::launch::async | std::launch::deferred : std::launch::deferred;
+}
+
 // Relative cost of a plan: per pass the HBM cost of its run length (in
 // place: reads and writes; relabelled: the writes only) times the fraction
 // of its tiles that a run from |0...0> launches (a tile whose rest qubits
@@ -2026,10 +2049,7 @@ static double plan_cost(const Plan& p, int amp_bytes)
     double c = 0.1 * (double)p.micro.size();
     for (size_t i = 0; i < p.passes.size(); i++) {
         const PassArgs& pa = p.passes[i];
-        double f = 1.0;
-        if ((int)i < p.support_passes && i < p.pass_zero.size())
-            for (int j = 0; j < pa.nrest; j++)
-                if ((p.pass_zero[i] >> pa.rest_pos[j]) & 1ull) f *= 0.5;
+        const double f = launched(p, i);
         // (a pass of the full op set is bound by its register steps; its
         // reads cost it what they cost in place)
         const bool relabelled = p.relabel_begin >= 0 && (long)i >= p.relabel_begin && (pa.light || pa.stream);
@@ -2038,12 +2058,87 @@ static double plan_cost(const Plan& p, int amp_bytes)
     return c;
 }
 
+// Cost of a plan's passes by what they run, for the choice between streamed
+// passes and register ops: in units of a copy of the state, 0.6 a pass, 0.06
+// a register step and the ops below.  Fitted on one MI355X to the passes of 25-
+// and 28-qubit circuits in both forms (complex128 and complex64 agree to a few
+// percent; standard error 0.05-0.1 of a copy a pass).
+static double form_cost(const Plan& p, bool zero_start)
+{
+    double c = 0;
+    for (size_t i = 0; i < p.passes.size(); i++) {
+        const PassArgs& pa = p.passes[i];
+        double t = 0.6;
+        for (uint32_t m = pa.micro_begin; m < pa.micro_begin + pa.micro_count; m++) {
+            const MicroStep& ms = p.micro[m];
+            t += 0.06;
+            for (uint32_t o = 0; pa.stream; o++) {
+                const uint32_t code = (p.raw[ms.op_begin + o / 4] >> (8 * (o % 4))) & 255u;
+                if (code == SC_END) break;
+                t += code == SC_LAYER ? 0.08 : code == SC_DIAG ? 0.05 : code >= SC_PHASE ? 0.04 : 0.033;
+            }
+            for (uint32_t o = 0; !pa.stream && o < ms.op_count; o++) {
+                const int kind = p.ops[ms.op_begin + o].code >> 8;
+                const bool kron = kind == OK_KRON || kind == OK_EKRON || kind == OK_FKRON;
+                t += kron ? 0.07 : kind == OK_DENSE ? 0.05 : 0.025;
+            }
+        }
+        c += t * (zero_start ? launched(p, i) : 1.0);
+    }
+    return c;
+}
+
+// Whether a program runs faster on streamed passes (k_stream) than on register
+// ops (k_pass).  Streams need far fewer passes where CRk gates tie many qubits
+// together, but each of their ops costs more than a register op that does the
+// same, so programs of few CRk gates among layers lose: both forms are planned
+// once, at one shape, and the streamed one has to be cheaper by 8 % both from
+// |0...0> and from a product state.  Predicted and measured ratios, streamed to
+// register ops, 28 qubits complex128 from a product state: QFT 0.23 and 0.27,
+// QFT behind 10 layers 0.53 and 0.64, 6 rounds of ring CRk and RX 0.83 and
+// 0.92, 10 layers with 256 CRk 0.91 and 0.98, with 64 CRk 1.00 and 1.03, with
+// 4 CRk 1.04 and 1.30, H and CNOT layers with 16 CRk 1.17 and 1.28.  Up to 20
+// qubits, where fewer launches count as well, it has to be no dearer (16
+// qubits, 800 random gates: 0.96 and 0.84), and a state of one tile, one
+// latency-bound pass in either form, is streamed up to a ratio of 1.2 (12
+// qubits: QFT 0.65 and 0.64, layers with one CRk 1.05 and 0.92, ring CRk 1.13
+// and 0.98, H and CNOT layers 1.30 and 1.04).
+static bool streams_pay(const Program& prog, const PlanOptions& opt)
+{
+    if (!opt.phases || opt.micro_bits != 4 || !Builder::streamable(prog)) return false;
+    PlanOptions o = opt;
+    o.weigh = o.reorder = o.auto_low = o.auto_tile = false;
+    if (opt.auto_tile) o.tile_bits = o.min_qubits = 12;
+    if (opt.auto_low) o.low_qubits = opt.amp_bytes == 16 ? 3 : 4;
+    Plan plans[2];
+    std::string errs[2];
+    auto plan = [&](int streamed) {
+        PlanOptions f = o;
+        f.stream = streamed;
+        errs[streamed] = build_plan(prog, f, plans[streamed]);
+    };
+    std::future<void> other = std::async(plan_launch(prog, opt), plan, 1);
+    plan(0);
+    other.get();
+    if (!errs[0].empty() || !errs[1].empty()) return errs[1].empty();
+    const double less = prog.nqubits <= 12 ? 1.2 : prog.nqubits <= 20 ? 1.0 : 0.92;
+    for (bool zero_start : {true, false})
+        if (!(form_cost(plans[1], zero_start) < less * form_cost(plans[0], zero_start))) return false;
+    return true;
+}
+
 std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
 {
     if (opt.split) {
         PlanOptions o = opt;
         o.split = false;
         return build_plan(split_kron_gates(prog), o, plan);
+    }
+    if (opt.stream && opt.weigh) {
+        PlanOptions o = opt;
+        o.weigh = false;
+        o.stream = streams_pay(prog, opt);
+        return build_plan(prog, o, plan);
     }
     if (opt.auto_tile) {
         // complex64 by default: 13-qubit tiles (64 KiB; 8 free tile qubits
@@ -2105,16 +2200,13 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
         bool have = false;
         const int lo = opt.amp_bytes == 16 ? 2 : 3;
         const int hi = std::min(lo + 3, std::min(opt.tile_bits, kMaxQubits) - opt.micro_bits);
-        // The candidates are independent: planned at the same time for
-        // programs whose planning (about 1 us a gate each) outweighs the
-        // start of a thread.
+        // The candidates are independent.
         struct Cand {
             Plan plan;
             std::string err;
         };
         std::vector<std::future<Cand>> cands;
-        const auto how = opt.threads && prog.gates.size() >= 256 ? std::launch::async | std::launch::deferred
-                                                                 : std::launch::deferred;
+        const auto how = plan_launch(prog, opt);
         for (int low = lo; low <= hi; low++) {
             o.low_qubits = low;
             cands.push_back(std::async(how, [&prog, o] {
@@ -2148,15 +2240,7 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
     if (opt.amp_bytes != 16 && opt.amp_bytes != 8) return "amplitudes have 8 or 16 bytes";
     if (opt.micro_bits != 4 && (opt.mfma || opt.mfma_fuse || opt.mfma5 || opt.gate_mfma)) return "matrix-core steps need 4-bit micro-steps";
     Builder b{prog, opt, plan};
-    if (opt.stream && opt.phases && opt.micro_bits == 4) {
-        // a program of gates that can all be streamed, CRk among them
-        bool all = true, crk = false;
-        for (const PlanGate& g : prog.gates) {
-            all = all && b.streamable(g);
-            crk = crk || g.id == 4;
-        }
-        b.phases = all && crk;
-    }
+    b.phases = opt.stream && opt.phases && opt.micro_bits == 4 && Builder::streamable(prog);
     b.zero = !opt.zero_start ? 0ull : plan.nq_int >= 64 ? ~0ull : ((1ull << plan.nq_int) - 1ull);
     // a pass with phases outside its tile has no other form
     auto without_phases = [&] {

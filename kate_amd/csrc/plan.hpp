@@ -211,7 +211,9 @@ struct PlanOptions {
     bool reorder = true;     // swap-free programs: also plan the gates in a canonical order, keep the cheaper
     bool scatter = false;    // 2+ trailing permutation passes become one out-of-place pass (needs a second buffer)
     bool relabel = false;    // with scatter: passes after the support region read contiguous tiles (relabelled qubits)
-    bool stream = false;     // streamed passes (k_stream) where every gate allows; 4-bit micro-steps only
+    bool stream = false;     // streamed passes (k_stream) for programs of 1-qubit, CNOT and CRk gates, CRk among
+                             // them; 4-bit micro-steps only
+    bool weigh = true;       // with stream: only where the streamed form is the cheaper one (streams_pay)
     bool phases = true;      // with stream: CRk gates need only one of their qubits in registers
     bool zero_start = true;  // the first pass sees |0...0> (false: any state, e.g. a product input; no support region)
 };
