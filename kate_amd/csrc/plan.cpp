@@ -322,6 +322,59 @@ Program split_kron_gates(const Program& in)
     return out;
 }
 
+// 32-bit words of a dense k-qubit gate's matrix-core operand.
+size_t operand_words(int k, int amp_bytes) { return ((size_t)4 << (2 * k)) * (size_t)amp_bytes / 8; }
+
+// A dense 2^k x 2^k complex matrix (row-major, interleaved) as the lane-
+// ordered A operand of an SK_MFMA step (kernels_dev.hpp mfma_gate), in the
+// state's precision: for contraction steps 2t + p, row block b and lane l,
+// the entry of the real embedding at gate row g = 4t + l/16, part p, and
+// the output row of index i = l%16: gate row 8b + 4(i/8) + i%4, part
+// (i/4)%2 (double) or gate row 8b + i/2, part i%2 (float).
+void lay_operand(const double* m, int k, bool f64, uint32_t* out)
+{
+    const int D = 1 << k, RB = 2 * D / 16, T = D / 4;
+    for (int t = 0; t < T; t++)
+        for (int b = 0; b < RB; b++)
+            for (int lane = 0; lane < 64; lane++) {
+                const int i = lane % 16, g = 4 * t + lane / 16;
+                const int row = f64 ? 8 * b + 4 * (i / 8) + i % 4 : 8 * b + i / 2;
+                const int part = f64 ? (i / 4) % 2 : i % 2;
+                const double* e = m + 2 * ((size_t)row * D + g);
+                const double v[2] = {part ? e[1] : e[0], part ? e[0] : -e[1]};
+                if (f64) {
+                    std::memcpy(out, v, 16);
+                    out += 4;
+                } else {
+                    const float f[2] = {(float)v[0], (float)v[1]};
+                    std::memcpy(out, f, 8);
+                    out += 2;
+                }
+            }
+}
+
+// Puts the matrix-core operands of the chosen plan where its steps expect them.
+void lay_operands(const Program& prog, int amp_bytes, Plan& plan)
+{
+    if (plan.operands.empty()) return;
+    std::vector<uint32_t> raw(plan.raw.size() + plan.operand_words);
+    size_t from = 0, at = 0;
+    auto words_up_to = [&](size_t end) {  // the words between the operands
+        std::copy(plan.raw.begin() + (long)from, plan.raw.begin() + (long)(from + end - at), raw.begin() + (long)at);
+        from += end - at;
+        at = end;
+    };
+    for (const GateOperand& o : plan.operands) {
+        words_up_to(o.at);
+        lay_operand(prog.mat.data() + 2 * o.moff, o.nbits, amp_bytes == 16, raw.data() + at);
+        at += operand_words(o.nbits, amp_bytes);
+    }
+    words_up_to(raw.size());
+    plan.raw.swap(raw);
+    plan.operands.clear();
+    plan.operand_words = 0;
+}
+
 struct Builder {
     const Program& prog;
     const PlanOptions& opt;
@@ -561,39 +614,29 @@ struct Builder {
         return "";
     }
 
-    // A dense 2^k x 2^k complex matrix (row-major, interleaved) as the lane-
-    // ordered A operand of an SK_MFMA step (kernels_dev.hpp mfma_gate), in the
-    // state's precision: for contraction steps 2t + p, row block b and lane l,
-    // the entry of the real embedding at gate row g = 4t + l/16, part p, and
-    // the output row of index i = l%16: gate row 8b + 4(i/8) + i%4, part
-    // (i/4)%2 (double) or gate row 8b + i/2, part i%2 (float).
-    uint32_t add_gate_operand(const double* m, int k)
+    // First word after what the plan has in Plan::raw, the operands that are not
+    // laid out yet included.
+    uint32_t raw_at() const { return (uint32_t)(plan.raw.size() + plan.operand_words); }
+
+    // The operand of a gate composed by the planner, laid out at once.
+    uint32_t add_window_operand(const double* m, int k)
     {
-        const int D = 1 << k, RB = 2 * D / 16, T = D / 4;
-        const bool f64 = opt.amp_bytes == 16;
-        while (plan.raw.size() % 4) plan.raw.push_back(0);  // 16-byte loads
-        const uint32_t off = (uint32_t)plan.raw.size();
-        for (int t = 0; t < T; t++)
-            for (int b = 0; b < RB; b++)
-                for (int lane = 0; lane < 64; lane++)
-                    for (int p = 0; p < 2; p++) {
-                        const int i = lane % 16, g = 4 * t + lane / 16;
-                        const int row = f64 ? 8 * b + 4 * (i / 8) + i % 4 : 8 * b + i / 2;
-                        const int part = f64 ? (i / 4) % 2 : i % 2;
-                        const double mr = m[2 * ((size_t)row * D + g)], mi = m[2 * ((size_t)row * D + g) + 1];
-                        const double v = part == p ? mr : (part == 0 ? -mi : mi);
-                        uint32_t w[2];
-                        if (f64) {
-                            std::memcpy(w, &v, 8);
-                            plan.raw.push_back(w[0]);
-                            plan.raw.push_back(w[1]);
-                        } else {
-                            const float f = (float)v;
-                            std::memcpy(w, &f, 4);
-                            plan.raw.push_back(w[0]);
-                        }
-                    }
-        return off;
+        while (raw_at() % 4) plan.raw.push_back(0);
+        const uint32_t at = raw_at();
+        const size_t n = plan.raw.size();
+        plan.raw.resize(n + operand_words(k, opt.amp_bytes));
+        lay_operand(m, k, opt.amp_bytes == 16, plan.raw.data() + n);
+        return at;
+    }
+
+    // Reserves an SK_MFMA step's operand; returns its place.
+    uint32_t add_gate_operand(size_t moff, int k)
+    {
+        while (raw_at() % 4) plan.raw.push_back(0);  // 16-byte loads
+        const uint32_t at = raw_at();
+        plan.operands.push_back({at, (uint8_t)k, moff});
+        plan.operand_words += operand_words(k, opt.amp_bytes);
+        return at;
     }
 
     static uint16_t bf16_rn(float f)
@@ -611,8 +654,9 @@ struct Builder {
     uint32_t add_bf16_operand(const double* m, int k)
     {
         const int D = 1 << k, RB = 2 * D / 32, T = 2 * D / 16;
-        const uint32_t off = (uint32_t)plan.raw.size();
-        plan.raw.resize(plan.raw.size() + (size_t)RB * T * 2 * 64 * 4);
+        const uint32_t at = raw_at();
+        const size_t off = plan.raw.size();
+        plan.raw.resize(off + (size_t)RB * T * 2 * 64 * 4);
         for (int rb = 0; rb < RB; rb++)
             for (int t = 0; t < T; t++)
                 for (int lane = 0; lane < 64; lane++) {
@@ -634,7 +678,7 @@ struct Builder {
                         for (int w = 0; w < 4; w++) dst[w] = (uint32_t)src[2 * w] | ((uint32_t)src[2 * w + 1] << 16);
                     }
                 }
-        return off;
+        return at;
     }
 
     // The matrix of gate g on the window bits `wb` (tile bits, ascending),
@@ -1215,11 +1259,11 @@ struct Builder {
     {
         pa.ops_begin = (uint32_t)plan.ops.size();
         pa.coef_begin = (uint32_t)(plan.coef.size() / 2);
-        pa.raw_begin = (uint32_t)plan.raw.size();
+        pa.raw_begin = raw_at();
         const std::string e = pack_micro_form(gl, tile_of, pa);
         pa.ops_end = (uint32_t)plan.ops.size();
         pa.coef_end = (uint32_t)(plan.coef.size() / 2);
-        pa.raw_end = (uint32_t)plan.raw.size();
+        pa.raw_end = raw_at();
         return e;
     }
 
@@ -1290,7 +1334,7 @@ struct Builder {
                 std::vector<double> u(2 * (size_t)(1 << w) * (1 << w), 0.0);
                 for (int d = 0; d < (1 << w); d++) u[2 * ((size_t)d * (1 << w) + d)] = 1.0;
                 for (int a : acc) compose_into(u, w, ms.bits, prog.gates[(size_t)rem[(size_t)a]], tile_of);
-                ms.coef = opt.mfma_bf16 ? add_bf16_operand(u.data(), w) : add_gate_operand(u.data(), w);
+                ms.coef = opt.mfma_bf16 ? add_bf16_operand(u.data(), w) : add_window_operand(u.data(), w);
                 fill_mfma_cols(ms, cols);
                 plan.micro.push_back(ms);
                 std::vector<int> next;
@@ -1338,7 +1382,7 @@ struct Builder {
                 ms.nbits = (uint8_t)g.k;
                 for (int i = 0; i < g.k; i++) ms.bits[i] = (uint8_t)tile_of[g.q[i]];
                 if (ms.kind == SK_MFMA || ms.kind == SK_MFMA_BF16) {
-                    ms.coef = ms.kind == SK_MFMA ? add_gate_operand(prog.mat.data() + 2 * g.moff, g.k)
+                    ms.coef = ms.kind == SK_MFMA ? add_gate_operand(g.moff, g.k)
                                                  : add_bf16_operand(prog.mat.data() + 2 * g.moff, g.k);
                     fill_mfma_cols(ms, cols);
                 } else {
@@ -2058,6 +2102,8 @@ static double plan_cost(const Plan& p, int amp_bytes)
     return c;
 }
 
+static std::string search_plan(const Program& prog, const PlanOptions& opt, Plan& plan);
+
 // Cost of a plan's passes by what they run, for the choice between streamed
 // passes and register ops: in units of a copy of the state, 0.6 a pass, 0.06
 // a register step and the ops below.  Fitted on one MI355X to the passes of 25-
@@ -2115,7 +2161,7 @@ static bool streams_pay(const Program& prog, const PlanOptions& opt)
     auto plan = [&](int streamed) {
         PlanOptions f = o;
         f.stream = streamed;
-        errs[streamed] = build_plan(prog, f, plans[streamed]);
+        errs[streamed] = search_plan(prog, f, plans[streamed]);
     };
     std::future<void> other = std::async(plan_launch(prog, opt), plan, 1);
     plan(0);
@@ -2127,18 +2173,13 @@ static bool streams_pay(const Program& prog, const PlanOptions& opt)
     return true;
 }
 
-std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
+static std::string search_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
 {
-    if (opt.split) {
-        PlanOptions o = opt;
-        o.split = false;
-        return build_plan(split_kron_gates(prog), o, plan);
-    }
     if (opt.stream && opt.weigh) {
         PlanOptions o = opt;
         o.weigh = false;
         o.stream = streams_pay(prog, opt);
-        return build_plan(prog, o, plan);
+        return search_plan(prog, o, plan);
     }
     if (opt.auto_tile) {
         // complex64 by default: 13-qubit tiles (64 KiB; 8 free tile qubits
@@ -2155,12 +2196,12 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
         o.auto_tile = false;
         o.tile_bits = 12;
         o.min_qubits = 12;
-        std::string e = build_plan(prog, o, plan);
+        std::string e = search_plan(prog, o, plan);
         if (!e.empty() || prog.nqubits < 13) return e;
         o.tile_bits = 13;
         o.min_qubits = 13;
         Plan alt;
-        if (!build_plan(prog, o, alt).empty()) return "";
+        if (!search_plan(prog, o, alt).empty()) return "";
         bool all_light = true;
         for (size_t i = 0; i < alt.passes.size(); i++)
             if (!alt.pass_is_remap[i] && alt.passes[i].micro_count && !alt.passes[i].light) all_light = false;
@@ -2170,12 +2211,12 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
     if (opt.reorder) {
         PlanOptions o = opt;
         o.reorder = false;
-        std::string e = build_plan(prog, o, plan);
+        std::string e = search_plan(prog, o, plan);
         bool swap_free = !prog.gates.empty();
         for (int k : prog.instr_kind) swap_free = swap_free && k == 1;
         if (!e.empty() || !swap_free) return e;
         Plan alt;
-        if (build_plan(canonical_order(prog), o, alt).empty() &&
+        if (search_plan(canonical_order(prog), o, alt).empty() &&
             plan_cost(alt, opt.amp_bytes) < plan_cost(plan, opt.amp_bytes))
             plan = std::move(alt);
         return "";
@@ -2211,7 +2252,7 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
             o.low_qubits = low;
             cands.push_back(std::async(how, [&prog, o] {
                 Cand c;
-                c.err = build_plan(prog, o, c.plan);
+                c.err = search_plan(prog, o, c.plan);
                 return c;
             }));
         }
@@ -2246,7 +2287,7 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
     auto without_phases = [&] {
         PlanOptions o = opt;
         o.phases = false;
-        return build_plan(prog, o, plan);
+        return search_plan(prog, o, plan);
     };
     std::vector<int> seg;
     size_t grp = 0;
@@ -2277,6 +2318,18 @@ std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
     if (opt.scatter) make_scatter(plan, opt.amp_bytes);
     if (opt.scatter && opt.relabel) make_relabel(plan);
     return "";
+}
+
+std::string build_plan(const Program& prog, const PlanOptions& opt, Plan& plan)
+{
+    if (opt.split) {
+        PlanOptions o = opt;
+        o.split = false;
+        return build_plan(split_kron_gates(prog), o, plan);
+    }
+    const std::string e = search_plan(prog, opt, plan);
+    if (e.empty()) lay_operands(prog, opt.amp_bytes, plan);
+    return e;
 }
 
 std::string Plan::describe(bool verbose) const

@@ -218,6 +218,14 @@ struct PlanOptions {
     bool zero_start = true;  // the first pass sees |0...0> (false: any state, e.g. a product input; no support region)
 };
 
+// A dense gate's matrix-core operand in Plan::raw, laid out once the plan is
+// chosen (candidate plans need only its place and size).
+struct GateOperand {
+    uint32_t at;     // first word
+    uint8_t nbits;
+    size_t moff;     // its matrix in Program::mat (complex elements)
+};
+
 struct Plan {
     int nq_int = 0;  // padded qubit count the kernels see
     int tile_bits = 0;
@@ -227,6 +235,8 @@ struct Plan {
     std::vector<MicroOp> ops;
     std::vector<double> coef;  // interleaved complex128; converted per dtype on upload
     std::vector<uint32_t> raw; // matrix-core operands and streamed op codes, uploaded bit for bit
+    std::vector<GateOperand> operands;  // of a candidate plan: not in `raw` yet, which holds the words between them
+    size_t operand_words = 0;
     std::vector<Phase> phases; // tile factors of the SC_PHASE ops, pass by pass
     int gate_passes = 0;
     int remap_passes = 0;
