@@ -178,6 +178,9 @@ int kate_batch_create(const kate_program* programs, int32_t count, const kate_op
         if (err.empty() && prog.nqubits > 32) err = "batched circuits have at most 32 qubits";
         kate::Plan plan;
         if (err.empty()) err = kate::build_plan(prog, po, plan);
+        // (the complex128 kernels may lack them: kValuSteps)
+        for (const kate::MicroStep& m : plan.micro)
+            if (m.kind == kate::SK_MFMA && po.amp_bytes == 16) err = "internal: matrix-core step in a complex128 batch";
         if (!err.empty()) {
             delete b;
             return bfail(KATE_ERR_PROGRAM, "circuit " + std::to_string(c) + ": " + err);

@@ -7,7 +7,7 @@ namespace kate {
 int launch_batch_kernel_f32(const BatchArgs& a, void* stream)
 {
     hipStream_t s = (hipStream_t)stream;
-    return a.wide ? batch_w<float, true>(a, s) : batch_w<float, false>(a, s);
+    return a.wide ? batch_w<float, kAnySteps>(a, s) : batch_w<float, kRegSteps>(a, s);
 }
 
 }  // namespace kate

@@ -7,7 +7,7 @@ namespace kate {
 int launch_batch_kernel_f64(const BatchArgs& a, void* stream)
 {
     hipStream_t s = (hipStream_t)stream;
-    return a.wide ? batch_w<double, true>(a, s) : batch_w<double, false>(a, s);
+    return a.wide ? batch_w<double, kAnySteps>(a, s) : batch_w<double, kRegSteps>(a, s);
 }
 
 }  // namespace kate

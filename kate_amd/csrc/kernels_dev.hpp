@@ -458,10 +458,10 @@ __device__ __forceinline__ void dense5(Cx<R>* tile, const MicroStep* __restrict_
 }
 
 // WIDE: kRegSteps instantiations run register steps only, kGateSteps ones also
-// SK_MFMA steps, kAnySteps ones every kind; keeping the larger steps out of the
-// common variants keeps their register counts at the waves per SIMD that LDS
-// allows.
-enum StepSet { kRegSteps = 0, kAnySteps = 1, kGateSteps = 2 };
+// SK_MFMA steps, kAnySteps ones every kind, kValuSteps ones all but matrix-core
+// steps; keeping the larger steps out of the common variants keeps their
+// register counts at the waves per SIMD that LDS allows.
+enum StepSet { kRegSteps = 0, kAnySteps = 1, kGateSteps = 2, kValuSteps = 3 };
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -828,12 +828,12 @@ __device__ __forceinline__ void run_steps(const PassArgs& pa, Cx<R>* tile, const
 #pragma unroll
             for (int s = 0; s < N; s++) lds_at(tile, bw ^ reg_offset<NB>(s, oc)) = v[s];
         } else if constexpr (WIDE != kRegSteps && NB == 4) {
-            const R* operand = reinterpret_cast<const R*>(raw + msp->coef);
-            const bool gate = WIDE == kGateSteps || msp->kind == SK_MFMA;
-            if (gate && msp->nbits == 5) mfma_gate<R, TB, NB, 5>(tile, msp, operand);
-            else if (gate && msp->nbits == 6) mfma_gate<R, TB, NB, 6>(tile, msp, operand);
-            else if (gate) mfma_gate<R, TB, NB, 4>(tile, msp, operand);
-            else if constexpr (WIDE == kAnySteps) {
+            if (WIDE == kGateSteps || (WIDE == kAnySteps && msp->kind == SK_MFMA)) {
+                const R* operand = reinterpret_cast<const R*>(raw + msp->coef);
+                if (msp->nbits == 5) mfma_gate<R, TB, NB, 5>(tile, msp, operand);
+                else if (msp->nbits == 6) mfma_gate<R, TB, NB, 6>(tile, msp, operand);
+                else mfma_gate<R, TB, NB, 4>(tile, msp, operand);
+            } else if constexpr (WIDE != kGateSteps) {
                 if (msp->kind == SK_MFMA_BF16) {
                     if constexpr (sizeof(R) == 4) {
                         if (msp->nbits == 5) mfma_bf16<TB, 5>(tile, msp, raw + msp->coef);
@@ -1643,7 +1643,13 @@ int batch_nb(const BatchArgs& a, hipStream_t s)
     if constexpr (sizeof(R) == 8)
         if (a.micro_bits == 3) return batch_t<R, TB, WIDE, 3>(a, s);
     if (a.micro_bits != 4) return (int)hipErrorInvalidValue;
-    return batch_t<R, TB, WIDE, 4>(a, s);
+    // A complex128 batch plans no matrix-core steps.  With their accumulators
+    // its kernels of 10- and 11-qubit tiles hold 318 registers, one wave per
+    // SIMD, without 254, two (256 circuits of 13-15 qubits with 8 dense
+    // 5-qubit gates each: 2.22 and 1.97 ms, 1.11 and 0.96 ms).  Those of 12
+    // qubits run one wave either way, and 8 % slower without (0.87, 0.94 ms).
+    constexpr int kSteps = sizeof(R) == 8 && WIDE && TB <= 11 ? (int)kValuSteps : WIDE;
+    return batch_t<R, TB, kSteps, 4>(a, s);
 }
 
 template <typename R, int WIDE>
