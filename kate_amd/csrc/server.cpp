@@ -177,7 +177,7 @@ constexpr unsigned kPlanners = 8;
 uint64_t round256(uint64_t x) { return (x + 255) & ~255ull; }
 
 // Footprint layout of a planned request inside its arena range.
-uint64_t layout(kate_server* s, Request& r)
+uint64_t layout(const kate_server* s, Request& r)
 {
     uint64_t o = 0;
     auto take = [&](uint64_t bytes) {
@@ -307,6 +307,12 @@ void plan_request(const kate_server* s, Request& r)
     std::string err;
     try {
         err = kate::build_plan(r.prog, po, r.plan);
+        // matrix-core operands are twice the size of the gates, and streamed
+        // steps carry tables: a request that only fits without runs without
+        if (err.empty() && layout(s, r) > (uint64_t)s->opt.hbm_budget_bytes) {
+            po.gate_mfma = po.stream = false;
+            err = kate::build_plan(r.prog, po, r.plan);
+        }
         if (err.empty() && s->opt.dtype == KATE_C64) r.coef32.assign(r.plan.coef.begin(), r.plan.coef.end());
         if (err.empty() && !r.theta_phi.empty()) product_factors(r);
     } catch (const std::exception& e) {
