@@ -1456,8 +1456,8 @@ int stream_r(int tile_bits, void* state, const PassArgs& pa, const DevPlan& dp, 
         (pa.phase_count && !dp.phases))
         return (int)hipErrorInvalidValue;
     // the planner streams only plans whose tile size it chose: 12 qubits, 10 or
-    // 11 for states that small, 13 for complex64 plans of light passes, whose
-    // permutations stay off k_stream
+    // 11 for states that small (13 only in complex64 plans of nothing but light
+    // passes)
     switch (tile_bits) {
     case 10: return stream_t<R, 10, WARM>(state, pa, dp, s);
     case 11: return stream_t<R, 11, WARM>(state, pa, dp, s);

@@ -2058,8 +2058,9 @@ static Program canonical_order(const Program& in)
 // writes runs of `run_bytes`, in the units of run_cost.  Fitted on one
 // MI355X, 30-qubit layered circuit: relabelled passes of s register steps
 // take about 0.5 + 0.1 s (complex128) and 0.67 + 0.11 s (complex64) times
-// an in-place 128 B-run copy, for 64 B write runs as for longer ones; 32 B
-// runs double some passes.
+// an in-place 128 B-run copy, for 64 B write runs as for longer ones (both
+// write whole lines, order_writes).  No candidate of the planner's has shorter
+// runs; those of a caller's low_qubits keep their price in place.
 static double relabel_run_cost(int run_bytes)
 {
     return run_bytes <= 32 ? 2.5 : 0.6;
@@ -2233,7 +2234,11 @@ static std::string search_plan(const Program& prog, const PlanOptions& opt, Plan
         // (30-qubit layered circuit, complex64 13-qubit tiles: 18 passes with
         // 3 low qubits 85.6 ms, 25 with 5 96.6 ms; complex128: 19 passes with
         // 2 low qubits 150.5 ms, 24 with 3 157.6 ms, both bound by their
-        // register steps more than by their lines).
+        // register steps more than by their lines).  6 low qubits in
+        // complex128 would be the cheapest by cost for a few circuits of one or
+        // two layers, none of which ran faster with them (20 qubits, 2 layers
+        // 77 us with 5 and 79 with 6; 28 qubits, 2 Haar layers 2.34 ms with 4
+        // and 2.38).
         PlanOptions o = opt;
         o.auto_low = false;
         std::string first_err;
