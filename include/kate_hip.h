@@ -347,7 +347,8 @@ int kate_batch_last_ms(const kate_batch* batch, float* ms);
  * requests in flight overlap on the device.  Each returns <Z_S> for up to 15
  * real-qubit masks (FP64 accumulation, normalised).  A request of 22 qubits
  * or more holds two state buffers in the arena (its passes run out of place,
- * relabelled); a smaller one holds one. */
+ * relabelled); a smaller one holds one.  A request whose plan exceeds the
+ * arena with matrix-core operands or streamed passes runs without them. */
 typedef struct kate_server_options {
     int32_t dtype;
     int32_t device;
